@@ -25,12 +25,9 @@
 namespace {
 
 constexpr int WCH = 128;          // K columns staged per chunk (4 k-steps)
-constexpr int WKS = WCH / 32;     // k-steps per chunk
 constexpr int WT = 2;             // 16-column tiles per wave: each operand read from LDS feeds WT multiplies
-constexpr int WRC = 1;            // chunks of fragments in flight per wave
-constexpr int WSPF = WRC * WKS * WT;   // fragment loads in flight per wave
+constexpr int WSPF = WCH / 32 * WT;    // fragment loads in flight per wave
 constexpr int WMAXR = 128;        // max activation rows of one expert in a wide group
-constexpr int WLDA = WCH + 8;     // LDS row stride (halves): rows of a chunk start on different banks
 
 struct WEx {
   const h16x8* w;      // packed weights: fragment (tile t, k-step s) at ((t * K/32) + s) * 64
@@ -67,8 +64,15 @@ struct WArgs {
 //              an XCD.
 enum { MAP_PLAIN = 0, MAP_PAIR = 1, MAP_XCD = 2 };
 
-template <int EPI, int NG, int WV>
+// CH: K columns staged per chunk.  WCH everywhere but in the folded cross attention's factor launches
+// (E_PART16, K split by head), whose k-splits are one head wide: the widest of 128, 64 and 32 that
+// divides the head width (320 at d = 2560: five chunks of 64).  A wave keeps the same WSPF
+// fragments in flight at every CH, over RC chunks.
+template <int EPI, int NG, int WV, int CH>
 __global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
+  constexpr int WKS = CH / 32;      // k-steps per chunk
+  constexpr int WRC = WCH / CH;     // chunks of fragments in flight per wave
+  constexpr int WLDA = CH + 8;      // LDS row stride (halves): rows of a chunk start on different banks
   extern __shared__ __align__(16) h16 lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int b = blockIdx.x;
@@ -97,13 +101,13 @@ __global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
   const WEx& ex = a.ex[e];
   const int S = ex.S;
   const int ksteps = a.K / 32;
-  const int KCW = a.K / a.ks, nsteps = KCW / 32, nchunk = KCW / WCH;
+  const int KCW = a.K / a.ks, nsteps = KCW / 32, nchunk = KCW / CH;
   const int t0 = (tg * WV + wave) * WT;               // this wave's WT adjacent 16-column tiles
   const int k0 = kc * KCW;
-  // staging of one chunk: vector idx = u * nt + thread, row idx / 16, columns (idx % 16) * 8 .. +7;
+  // staging of one chunk: vector idx = u * nt + thread, row idx / NVR, columns (idx % NVR) * 8 .. +7;
   // indices past the rows re-read the last vector (every load unconditional, see Stage)
   constexpr int NT = WV * 64;
-  constexpr int NVR = WCH / 8;                        // 16-byte vectors per row of a chunk
+  constexpr int NVR = CH / 8;                         // 16-byte vectors per row of a chunk
   constexpr int NSV = (NG * 16 * NVR + NT - 1) / NT;  // vectors per thread at the most rows
   const int total = S * NVR;
   // each staging slot's element offset in the operand, the same at every chunk (a gathered row's
@@ -118,7 +122,7 @@ __global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
   }
   h16x8 st[NSV];
   auto load_chunk = [&](int c) {
-    const h16* base = ex.a + k0 + c * WCH;
+    const h16* base = ex.a + k0 + c * CH;
 #pragma unroll
     for (int u = 0; u < NSV; ++u) st[u] = *(const h16x8*)(base + soff[u]);
   };
@@ -248,31 +252,31 @@ __global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
   }
 }
 
-size_t wide_lds(int S_max) { return (size_t)2 * S_max * WLDA * 2; }
+size_t wide_lds(int S_max, int ch) { return (size_t)2 * S_max * (ch + 8) * 2; }
 
-template <int EPI, int NG, int WV>
+template <int EPI, int NG, int WV, int CH>
 int launch_wide_k(const WArgs& a, size_t lds, hipStream_t st) {
   static unsigned long long attr_set = 0;
   int dev = 0;
   CFH_HIP(hipGetDevice(&dev));
   if (dev < 64 && !(attr_set & (1ull << dev))) {
-    CFH_HIP(hipFuncSetAttribute((const void*)k_wide<EPI, NG, WV>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    CFH_HIP(hipFuncSetAttribute((const void*)k_wide<EPI, NG, WV, CH>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 150 * 1024));
     attr_set |= 1ull << dev;
   }
   const long long wgs = (long long)a.nex * a.ks * a.wg_per_kc;
-  hipLaunchKernelGGL((k_wide<EPI, NG, WV>), dim3((unsigned)wgs), dim3(WV * 64), lds, st, a);
+  hipLaunchKernelGGL((k_wide<EPI, NG, WV, CH>), dim3((unsigned)wgs), dim3(WV * 64), lds, st, a);
   CFH_LAUNCH_CHECK();
   return CFH_OK;
 }
 
 // Shape checks of a wide launch (also used by the plan): CFH_OK when every unit of wv waves covers
 // whole tiles, every k-split a whole number of chunks, and the rows fit.
-int wide_check(const WArgs& a, int wv, int S_max) {
-  if (a.nex < 1 || a.nex > 4 || a.N <= 0 || a.N % 16 || a.ks <= 0 || a.K % a.ks || (a.K / a.ks) % WCH)
+int wide_check(const WArgs& a, int wv, int S_max, int ch = WCH) {
+  if (a.nex < 1 || a.nex > 4 || a.N <= 0 || a.N % 16 || a.ks <= 0 || a.K % a.ks || (a.K / a.ks) % ch)
     return CFH_E_UNSUPPORTED;
   if ((wv != 4 && wv != 6 && wv != 8 && wv != 12) || (a.N / 16) % (WT * wv) || S_max < 1 || S_max > WMAXR ||
-      wide_lds(S_max) > 150 * 1024)
+      wide_lds(S_max, ch) > 150 * 1024)
     return CFH_E_UNSUPPORTED;
   if (a.pair && a.nex % 2) return CFH_E_UNSUPPORTED;
   return CFH_OK;
@@ -298,12 +302,12 @@ int wide_wv(int tiles, int units) {
 }
 
 
-template <int EPI>
+template <int EPI, int CH = WCH>
 int launch_wide(const WArgs& a0, int wv, hipStream_t st) {
   WArgs a = a0;
   int S_max = 0;
   for (int e = 0; e < a.nex; ++e) S_max = std::max(S_max, a.ex[e].S);
-  if (wide_check(a, wv, S_max)) return CFH_E_UNSUPPORTED;
+  if (wide_check(a, wv, S_max, CH)) return CFH_E_UNSUPPORTED;
   for (int e = 0; e < a.nex; ++e)
     if (a.ex[e].S < 1 || a.ex[e].lda < a.K || !a.ex[e].w || !a.ex[e].a || !a.ex[e].out) return CFH_E_INVALID;
   a.wg_per_kc = (a.N / 16) / (WT * wv);
@@ -314,19 +318,27 @@ int launch_wide(const WArgs& a0, int wv, hipStream_t st) {
     a.map = MAP_XCD;
   else
     a.map = pair_runs ? MAP_PAIR : MAP_PLAIN;
-  const size_t lds = wide_lds(S_max);
+  const size_t lds = wide_lds(S_max, CH);
   const int ng = (S_max + 15) / 16;
+  // (the factor launches come in 4-wave workgroups only)
+  if constexpr (EPI == E_PART16) {
+    if (wv != 4) return CFH_E_UNSUPPORTED;
+    if (ng <= 2) return launch_wide_k<EPI, 2, 4, CH>(a, lds, st);
+    if (ng <= 4) return launch_wide_k<EPI, 4, 4, CH>(a, lds, st);
+    return launch_wide_k<EPI, 8, 4, CH>(a, lds, st);
+  } else {
 #define CFH_WIDE(G)                                                                 \
   if (ng <= G) {                                                                    \
     switch (wv) {                                                                   \
-      case 4: return launch_wide_k<EPI, G, 4>(a, lds, st);                          \
-      case 6: return launch_wide_k<EPI, G, 6>(a, lds, st);                          \
-      case 8: return launch_wide_k<EPI, G, 8>(a, lds, st);                          \
-      default: return launch_wide_k<EPI, G, 12>(a, lds, st);                        \
+      case 4: return launch_wide_k<EPI, G, 4, CH>(a, lds, st);                          \
+      case 6: return launch_wide_k<EPI, G, 6, CH>(a, lds, st);                          \
+      case 8: return launch_wide_k<EPI, G, 8, CH>(a, lds, st);                          \
+      default: return launch_wide_k<EPI, G, 12, CH>(a, lds, st);                        \
     }                                                                               \
   }
   CFH_WIDE(2) CFH_WIDE(4) CFH_WIDE(8)
 #undef CFH_WIDE
+  }
   return CFH_E_UNSUPPORTED;
 }
 

@@ -785,6 +785,7 @@ struct Plan {
                       // rows in one XBLK launch (k_xblock) instead of three
   bool wide;          // more than two requests a group: every row of the group shares each weight
                       // stream through the chunked-staging kernels (cfh_wide.h)
+  int fold_ch;        // wide, folded: K columns a staging chunk of the factor launches (fold_chunk)
   WideShape ws[2];    // wide launch shapes for one group a launch, and for two (ws[1].ok: a batch of
                       // several groups runs two at a time, both groups' entries in every launch)
   bool ok;
@@ -810,6 +811,23 @@ int wide_wv_resident(int tiles, int units) {
     }
   }
   return best ? best : wide_wv(tiles, units);
+}
+
+// Staging chunk of the wide factor launches: the widest that divides a head.
+int fold_chunk(int hd) {
+  for (int ch : {128, 64, 32})
+    if (hd % ch == 0) return ch;
+  return 0;
+}
+
+// The factor launch with its staging chunk.
+int launch_wide_fold(const WArgs& a, int ch, hipStream_t st) {
+  switch (ch) {
+    case 128: return launch_wide<E_PART16, 128>(a, 4, st);
+    case 64: return launch_wide<E_PART16, 64>(a, 4, st);
+    case 32: return launch_wide<E_PART16, 32>(a, 4, st);
+    default: return CFH_E_UNSUPPORTED;
+  }
 }
 
 // Wide launch shapes for `groups` request groups a launch: about one workgroup per CU for each
@@ -855,7 +873,7 @@ WideShape wide_shape(const Plan& p, int groups) {
          !wide_check(wa(p.d, p.d, s.ks_wo, units), s.wv_split, p.Smax) &&
          !wide_check(wa(p.d, p.fd, s.ks_ww2, units), s.wv_split, p.Smax) &&
          !wide_check(wa(p.d, p.d, s.ks_wout, units), s.wv_split, p.Smax) &&
-         (p.fold ? !wide_check(wa(p.d, p.d, p.H, groups * p.nch), 4, p.Ct)
+         (p.fold ? !wide_check(wa(p.d, p.d, p.H, groups * p.nch), 4, p.Ct, p.fold_ch)
                  : s.ks_oc > 0 && !wide_check(wa(p.d, p.d, 1, units), s.wv_qc, p.Smax) &&
                        !wide_check(wa(p.d, p.d, s.ks_oc, units), s.wv_split, p.Smax));
   return s;
@@ -869,9 +887,13 @@ void make_wide_plan(Plan& p, const cfh_flow_dims* dm) {
   p.fold2 = false;
   p.ks_fold = p.H;
   p.S_fold = p.Ct;
-  // the cross attention folded (one head a k-chunk: its factors split-K by head need head widths
-  // of whole staging chunks) or unfolded (q projection, attention per (request, head), out-proj)
-  p.ok = (p.fold ? p.hd % WCH == 0 : p.hd % 8 == 0) && p.d % WCH == 0 && p.fd % WCH == 0 &&
+  // the cross attention folded (one head a k-chunk: its factors split-K by head, in staging chunks
+  // that divide the head width) or unfolded (q projection, attention per (request, head), out-proj).
+  // Head widths of 128 used to be the only folded ones here, and every other folded width (d = 2560:
+  // 320) drafted a batch two requests a weight stream: 13 requests at d = 2560 took 53.4 ms a flow
+  // pass, 12.7 ms as one wide group.
+  p.fold_ch = p.fold ? fold_chunk(p.hd) : 0;
+  p.ok = (p.fold ? p.fold_ch > 0 : p.hd % 8 == 0) && p.d % WCH == 0 && p.fd % WCH == 0 &&
          p.Smax <= WMAXR && p.Ct <= WMAXR && p.C <= 8 && 2 * p.KD <= MAXR && res_nq(p.d) > 0;
   if (!p.ok) return;
   p.ws[0] = wide_shape(p, 1);
@@ -1473,7 +1495,7 @@ int per_draft_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout& 
             x.pack = q == 0;
           }
         }
-      if ((rc = launch_wide<E_PART16>(a, 4, st))) return rc;
+      if ((rc = launch_wide_fold(a, p.fold_ch, st))) return rc;
     }
   return CFH_OK;
 }

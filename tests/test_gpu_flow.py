@@ -208,11 +208,11 @@ def test_packed_batch_matches_oracle_per_request(cuda, d, B, layers):
     """A batch drafts in groups whose rows share every weight stream: two requests a 16-row tile
     (attention masked to each request's own rows and context), or, above two requests, wide groups
     of up to 16 requests (rows staged in K chunks, self attention per request; the cross attention
-    folded in subgroups of two where the head width is a multiple of 128, else unfolded: q
+    folded in subgroups of two where the head width is a multiple of 32, else unfolded: q
     projection, attention per request and head, out-projection); two wide groups at a time share
     every launch.  Each request's hiddens against the oracle on its own context, and against the
-    same request drafted alone in the same numerics.  d = 512 (head width 64) keeps the two-request
-    tiles, B = 5 ending with a group of one; d = 640 (head width 80) runs B = 3 as one unfolded wide
+    same request drafted alone in the same numerics.  d = 512 (head width 64): B = 2 a two-request
+    tile, B = 5 one wide group; d = 640 (head width 80) runs B = 3 as one unfolded wide
     group and B = 20 as two; d = 1024: B = 3 one wide group of an odd request count, B = 21 two (11
     and 10 requests), B = 40 a pair of 14-request groups then one of 12."""
     cfg = flownet(d, layers=layers, flow_steps=2)
@@ -233,6 +233,27 @@ def test_packed_batch_matches_oracle_per_request(cuda, d, B, layers):
         print(f"  request {b}: vs oracle {e:.3e}, vs drafted alone {es:.3e}", flush=True)
         assert np.isfinite(to64(z[b:b + 1])).all()
         assert e < TOL_FP16 and es < TOL_FP16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,B", [(256, 3), (768, 17), (2560, 5)])
+def test_wide_groups_of_other_head_widths_match_oracle(cuda, d, B):
+    """Folded wide groups whose head width is not a multiple of 128: the factors' split-K by head runs
+    in staging chunks of 32 columns (head width 32: one chunk; 96: three, of which the fragment ring
+    holds four) or 64 (320: five, an odd count).  768 x 17 also pairs two groups (9 and 8 requests)
+    in every launch.  Each request against the oracle on its own context."""
+    cfg = flownet(d, layers=1, flow_steps=2)
+    assert plan_flags(cfg, B) & (_lib.PLAN_WIDE | _lib.PLAN_FOLD) == _lib.PLAN_WIDE | _lib.PLAN_FOLD
+    W = _flow_weights(cfg, seed=17)
+    ctx = synthetic_context(B, cfg.context_size, d, seed=23)
+    print(f"[flow wide] d={d} B={B}", flush=True)
+    ff = FusedFlow(cfg, {k: v.to(cuda) for k, v in W.items()}, device=cuda)
+    z = ff.predict_hidden(ctx.to(cuda))
+    torch.cuda.synchronize()
+    ref = oflow.predict_hidden(weights64(W), to64(ctx), _ocfg(cfg), numerics="fp16_modules")
+    e = [rel_err(to64(z[b:b + 1]), ref[b:b + 1]) for b in range(B)]
+    print(f"  worst request {max(e):.3e}", flush=True)
+    assert np.isfinite(to64(z)).all() and max(e) < TOL_FP16
 
 
 @pytest.mark.gpu
