@@ -27,8 +27,27 @@ __device__ __forceinline__ f32x4 mfma_f16(h16x8 a, h16x8 b, f32x4 c) {
 
 __device__ __forceinline__ float r16(float x) { return (float)(h16)x; }
 
+// erf-GELU x Phi(x), Phi the normal distribution: the tail Phi(-|x|) = t P(t) exp(-x^2 / 2) with
+// t = 1 / (1 + 0.3 |x| / sqrt(2)) and P the degree-8 polynomial that minimises the largest relative
+// error for |x| <= 13.4 (Lawson's reweighted least squares against scipy's erfcx; 1.9e-8), and
+// Phi(|x|) = 1 - that.  About 20 instructions and no branch, where erff runs two divergent branches:
+// the batched up-projections went 41.4 -> 35.8 us (156 rows, d = 2560), 113 -> 107 us (384 rows,
+// d = 4096) and 20.1 -> 15.4 us (324 rows, d = 640).  The tail keeps its relative precision, which
+// 1 + erff loses to cancellation: over |x| <= 12 in float32, 4.8% of the fp16-rounded results of
+// 0.5 x (1 + erff(x / sqrt 2)) differ from the exact value's, 0.006% of these.
 __device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f));
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.21213203435596423f, fabsf(x), 1.0f));
+  float p = -0.06471702456474304f;
+  p = fmaf(p, t, 0.2425481528043747f);
+  p = fmaf(p, t, -0.2556130886077881f);
+  p = fmaf(p, t, 0.27319735288619995f);
+  p = fmaf(p, t, -0.04681551828980446f);
+  p = fmaf(p, t, 0.10721809417009354f);
+  p = fmaf(p, t, 0.07424122840166092f);
+  p = fmaf(p, t, 0.08534596860408783f);
+  p = fmaf(p, t, 0.08459480851888657f);
+  const float q = p * t * __builtin_amdgcn_exp2f(x * x * -0.72134752044448170368f);
+  return x * (x < 0.f ? q : 1.0f - q);
 }
 
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
