@@ -176,6 +176,66 @@ def test_gdn_vllm_form_matches_oracle(cuda, H, HV, state_dtype):
     assert np.array_equal(got_s[1], st[1].float().numpy())           # the prefix slot is only read
 
 
+def _random_parents(n, roots, seed):
+    rng = np.random.default_rng(seed)
+    return np.array([-1] * roots + [int(rng.integers(0, i)) for i in range(roots, n)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parent,V,state_dtype", [
+    (np.array([-1]), 64, torch.float32),                          # one node, one 64-row slice
+    (np.arange(-1, 15), 128, torch.float32),                      # one path of 16: one whole staging batch
+    (np.arange(-1, 16), 64, torch.bfloat16),                      # 17: a second batch of one step
+    (np.arange(-1, 33), 64, torch.float32),                       # 34: three batches
+    (_random_parents(100, 3, 4), 64, torch.bfloat16),             # chains ending at any depth, a forest
+    (_random_parents(256, 200, 5), 64, torch.float32),            # the most nodes, most of them leaves
+])
+def test_gdn_vllm_chains_match_oracle(cuda, parent, V, state_dtype):
+    """The serving form's chains (one per leaf, each node in the chain of its lowest child): every
+    node's output and state written once, whatever the chain it lies in and the staging batch its
+    step falls in.  Bounds as in test_gdn_vllm_form_matches_oracle."""
+    from chain_flow_amd.gdn import tree_gdn_vllm
+    N, H, HV, K = len(parent), 2, 4, 128
+    X, a, b, A_log, dt_bias, st = _vllm_inputs(N, H, HV, K, V, 31, state_dtype)
+    slots = torch.from_numpy(np.random.default_rng(6).permutation(N).astype(np.int32) + 2)
+    st_d = st.to(cuda)
+    print(f"[gdn vllm chains] N={N} V={V} {state_dtype}", flush=True)
+    o = tree_gdn_vllm(X.to(cuda), a.to(cuda), b.to(cuda), A_log, dt_bias, st_d, slots, torch.tensor(parent),
+                      num_q_heads=H)
+    torch.cuda.synchronize()
+    bf = state_dtype == torch.bfloat16
+    ro, rs = ogdn.tree_gdn_vllm(X.float().numpy(), a.float().numpy(), b.float().numpy(), A_log.numpy(),
+                                dt_bias.numpy(), st.float().numpy(), slots.numpy(), parent, 1, H, HV, K, V,
+                                K ** -0.5, state_bf16=bf, form="slots")
+    es = rel_err(st_d.float().cpu().numpy(), rs)
+    eo = rel_err(o.float().cpu().numpy(), ogdn._round_bf16(ro))
+    print(f"  out err {eo:.2e} state err {es:.2e}", flush=True)
+    assert es < (5e-4 if bf else 1e-5)
+    assert eo < 2e-3
+
+
+@pytest.mark.gpu
+def test_gdn_vllm_refuses_non_bfs_order(cuda):
+    """Node 2's parent does not precede it: NaN for it and for its descendants, their slots
+    unwritten; every other node as in a tree without them."""
+    from chain_flow_amd.gdn import tree_gdn_vllm
+    N, H, K, V = 6, 2, 128, 64
+    X, a, b, A_log, dt_bias, st = _vllm_inputs(N, H, H, K, V, 14, torch.bfloat16)
+    slots = torch.arange(2, N + 2, dtype=torch.int32)
+    args = (X.to(cuda), a.to(cuda), b.to(cuda), A_log, dt_bias)
+    st_g, st_b = st.to(cuda), st.to(cuda)
+    print("[gdn vllm non-bfs] 6 nodes", flush=True)
+    og = tree_gdn_vllm(*args, st_g, slots, torch.tensor([-1, 0, -1, 1, 2, 4]), num_q_heads=H)
+    ob = tree_gdn_vllm(*args, st_b, slots, torch.tensor([-1, 0, 3, 1, 2, 4]), num_q_heads=H)
+    torch.cuda.synchronize()
+    bad, keep = [2, 4, 5], [0, 1, 3]
+    assert torch.isnan(ob[bad].float()).all() and torch.equal(ob[keep], og[keep])
+    for n in keep:
+        assert torch.equal(st_b[n + 2], st_g[n + 2])
+    for n in bad:
+        assert torch.equal(st_b[n + 2].cpu(), st[n + 2])
+
+
 @pytest.mark.gpu
 def test_gdn_vllm_fp32_states_equal_research_kernel(cuda):
     """With fp32 slots and one q/k head per value head the serving kernel is the research kernel
