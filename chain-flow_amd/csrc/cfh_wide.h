@@ -4,14 +4,21 @@
 // chunk expert at draft_length 8) whose rows all multiply each packed weight fragment as it
 // streams past, so a group costs about one draft's weight traffic instead of one per two drafts.
 // The narrow streaming kernel (cfh_stream.h) stages its whole K chunk once and holds at most 16
-// rows; here the activation rows are staged in K chunks of WCH columns through two LDS buffers,
+// rows; here the activation rows are staged in K chunks of WCH columns through three LDS buffers,
 // refilled while the weights stream:
 //
-//   chunk c:  issue the loads of chunk c+1's rows into registers (they return after the weight
-//             fragments already in flight, which the multiplies need first anyway)
-//             multiply the chunk's WCH/32 k-steps of fragments, each against every 16-row group
-//             of the rows in LDS
-//             place chunk c+1's rows in the other buffer, one LDS barrier
+//   chunk c:  multiply the chunk's WCH/32 k-steps of fragments, each against every 16-row group of the
+//             rows in LDS; the rows of a k-step are read while the one before multiplies, those of
+//             the chunk's last k-step's successor from chunk c + 1's buffer, complete since the last
+//             barrier, so that neither the barrier nor the LDS latency stands before a multiply
+//             place chunk c + 2's rows (loaded during chunk c - 2) in the buffer chunk c - 1 left
+//             issue the loads of chunk c + 4's rows into the registers just freed
+//             one LDS barrier
+//
+// What bounds it (13 requests at d = 2560, the 157 MB up-projection, 35 us): copies of the kernel with
+// one part each taken out run at 24 us with the matrix instructions alone (no rows, no weights: about
+// 14 ns each a SIMD), 25 us with the rows' LDS reads too, 33 us with the rows' staging, 35 us
+// with the weights; of these 2 us are the launch, 1 us its start, 2-5 us the epilogue's stores.
 //
 // A wave owns WT adjacent 16-column tiles of one (expert, k-split) unit and keeps one accumulator
 // per (tile, 16-row group).  Self attention, which the narrow kernel computes while staging, runs as its own
@@ -19,14 +26,13 @@
 // once per draft into rows the cross K/V stream reads.
 #pragma once
 #include <algorithm>
+#include <type_traits>
 
 #include "cfh_stream.h"
 
 namespace {
 
 constexpr int WCH = 128;          // K columns staged per chunk (4 k-steps)
-constexpr int WT = 2;             // 16-column tiles per wave: each operand read from LDS feeds WT multiplies
-constexpr int WSPF = WCH / 32 * WT;    // fragment loads in flight per wave
 constexpr int WMAXR = 128;        // max activation rows of one expert in a wide group
 
 struct WEx {
@@ -66,15 +72,202 @@ enum { MAP_PLAIN = 0, MAP_PAIR = 1, MAP_XCD = 2 };
 
 // CH: K columns staged per chunk.  WCH everywhere but in the folded cross attention's factor launches
 // (E_PART16, K split by head), whose k-splits are one head wide: the widest of 128, 64 and 32 that
-// divides the head width (320 at d = 2560: five chunks of 64).  A wave keeps the same WSPF
-// fragments in flight at every CH, over RC chunks.
-template <int EPI, int NG, int WV, int CH>
-__global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
+// divides the head width (320 at d = 2560: five chunks of 64).  A wave keeps RC 128-column chunks of
+// fragments in flight at every CH.
+template <int I, int N, typename F>
+__device__ __forceinline__ void unrolled(F&& f) {   // f(0), f(1), .. f(N - 1), each a compile-time constant
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unrolled<I + 1, N>(f);
+  }
+}
+
+// LDS rows of one staged chunk: the NG row groups, rounded up to whole passes of the workgroup's threads.
+constexpr int wide_rows(int ng, int wv, int ch) {
+  const int rpv = wv * 64 / (ch / 8);
+  return (ng * 16 + rpv - 1) / rpv * rpv;
+}
+
+template <int EPI, int NG, int WV, int CH, int WT, int RS, int RC, bool GA>
+__device__ __forceinline__ void wide_unit(const WArgs& a, const WEx& ex, int kc, int tg) {
   constexpr int WKS = CH / 32;      // k-steps per chunk
-  constexpr int WRC = WCH / CH;     // chunks of fragments in flight per wave
+  constexpr int WRC = RC * WCH / CH;     // chunks of fragments in flight per wave
+  constexpr int WSPF = WRC * WKS * WT;   // fragment loads in flight per wave
+  // AP: a k-step's rows are read while the one before multiplies.  Eight-wave workgroups have no
+  // registers for it, and two waves a SIMD that cover the reads for each other.
+  constexpr bool AP = WKS % 2 == 0 && WV <= 4;
   constexpr int WLDA = CH + 8;      // LDS row stride (halves): rows of a chunk start on different banks
   extern __shared__ __align__(16) h16 lds[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // (the wave index read as a scalar keeps the weight pointers out of the vector registers)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int S = ex.S;
+  const int ksteps = a.K / 32;
+  const int KCW = a.K / a.ks, nsteps = KCW / 32, nchunk = KCW / CH;
+  // wave w: columns' share w % WC (WT adjacent 16-column tiles), rows' share w / WC (NGW of the NG groups)
+  constexpr int WC = WV / RS, NGW = NG / RS;
+  const int t0 = (tg * WC + wave % WC) * WT, g0 = wave / WC * NGW;
+  const int k0 = kc * KCW;
+  // staging of one chunk: thread t's vector u is row t / NVR + u NT / NVR, columns (t % NVR) * 8 .. +7;
+  // rows past S repeat the last one (every load unconditional, see Stage; the LDS rows they fill
+  // only reach output rows that are never stored)
+  constexpr int NT = WV * 64;
+  constexpr int NVR = CH / 8;                         // 16-byte vectors per row of a chunk
+  constexpr int RPV = NT / NVR;                       // rows between a thread's vectors
+  constexpr int NSV = (NG * 16 + RPV - 1) / RPV;      // vectors per thread
+  static_assert(NSV * RPV == wide_rows(NG, WV, CH), "LDS rows of a chunk");
+  const int trow = (int)threadIdx.x / NVR, tcol = (int)threadIdx.x % NVR;
+  // each vector's byte offset in the operand, the same at every chunk (a gathered row's
+  // index is read once)
+  typename std::conditional<GA, size_t, unsigned>::type soff[NSV];
+#pragma unroll
+  for (int u = 0; u < NSV; ++u) {
+    const int i = min(trow + u * RPV, S - 1);
+    if constexpr (GA) soff[u] = (size_t)max(ex.ids[(size_t)i * ex.ids_stride], 0) * ex.lda * 2 + tcol * 16;
+    else soff[u] = (unsigned)(i * ex.lda * 2 + tcol * 16);
+  }
+  h16x8 st0[NSV], st1[NSV];                           // rows of two chunks on their way to LDS
+  auto load_chunk = [&](int c, h16x8 (&st)[NSV]) {
+    const char* base = (const char*)(ex.a + k0 + c * CH);
+#pragma unroll
+    for (int u = 0; u < NSV; ++u) st[u] = *(const h16x8*)(base + soff[u]);
+  };
+  h16* const wbuf = lds + trow * WLDA + tcol * 8;
+  constexpr int BUF = NSV * RPV * WLDA;               // halves of one chunk buffer, of three
+  auto place_chunk = [&](int off, const h16x8 (&st)[NSV]) {
+#pragma unroll
+    for (int u = 0; u < NSV; ++u) *(h16x8*)(wbuf + off + u * (RPV * WLDA)) = st[u];
+  };
+  // the wave's fragments, k-step by k-step, the WT tiles of a k-step together; past the last
+  // k-step the pointers stay there, so the ring's surplus refills re-read lines just fetched
+  const char* lw = (const char*)(ex.w + ((size_t)t0 * ksteps + (size_t)kc * nsteps) * 64);
+  const size_t tstride = (size_t)ksteps * 1024;       // bytes to the next tile, same k-step
+  const unsigned loff = lane * 16;
+  int lleft = nsteps;
+  auto issue = [&](int u) -> h16x8 {
+    const h16x8 v = __builtin_nontemporal_load((const h16x8*)(lw + u * tstride + loff));
+    if (u == WT - 1) {
+      const bool adv = lleft > 1;
+      lw += adv ? 1024 : 0;
+      lleft -= adv;
+    }
+    return v;
+  };
+  // the products are taken as weights x rows: lane l's accumulator q is row l % 16 of the group, column
+  // cbase + q of the tile, so that a lane stores four adjacent columns at once
+  const int row = lane & 15, kg = lane >> 4, cbase = 4 * kg;
+  h16x4 bias[WT];
+  if constexpr (EPI == E_BIAS16 || EPI == E_GELU16) {
+#pragma unroll
+    for (int u = 0; u < WT; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bias[u][q] = ex.bias[(t0 + u) * 16 + cbase + q];   // (any alignment)
+  }
+  // operand chunks 0 and 1 first, then the weight prefetch (independent of them), then chunks 2 and 3
+  h16x8 ring[WSPF];
+  {
+    h16x8 p0[NSV], p1[NSV];
+    load_chunk(0, p0);
+    load_chunk(min(1, nchunk - 1), p1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < WSPF; ++p) {
+      ring[p] = issue(p % WT);
+      // issued in slot order: each multiply then waits for its own slot alone (with the order left
+      // free, slot 0 went out seventh and the first multiply waited for the whole ring)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    load_chunk(min(2, nchunk - 1), st0);
+    load_chunk(min(3, nchunk - 1), st1);
+    __builtin_amdgcn_sched_barrier(0);
+    place_chunk(0, p0);
+    place_chunk(BUF, p1);
+  }
+  lds_barrier();
+  f32x4 acc[WT][NGW];
+#pragma unroll
+  for (int u = 0; u < WT; ++u)
+#pragma unroll
+    for (int g = 0; g < NGW; ++g) acc[u][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  // (every row group is multiplied, which keeps the loop free of branches)
+  const h16* const rbuf = lds + (g0 * 16 + row) * WLDA + kg * 8;
+  int off0 = 0, off1 = BUF, off2 = 2 * BUF;           // buffers of chunks c, c + 1, c + 2
+  h16x8 av[AP ? 2 : 1][NGW];
+  auto read = [&](int off, int q, int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < NGW; ++g) av[set][g] = *(const h16x8*)(rbuf + off + g * (16 * WLDA) + q * 32);
+  };
+  if constexpr (AP) read(0, 0, 0);
+  constexpr int CYC = WRC % 2 ? 2 * WRC : WRC;        // chunks per ring cycle, an even count
+  auto chunk = [&](int c, auto hc) __attribute__((always_inline)) {
+    constexpr int h = decltype(hc)::value;            // c % CYC
+    constexpr int hs = h % WRC * WKS;
+#pragma unroll
+    for (int q = 0; q < WKS; ++q) {
+      if constexpr (AP) {
+        if (q + 1 < WKS) read(off0, q + 1, (q + 1) & 1);
+        else read(off1, 0, 0);                        // (past the last chunk: never used)
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        read(off0, q, 0);
+      }
+#pragma unroll
+      for (int g = 0; g < NGW; ++g) {
+#pragma unroll
+        for (int u = 0; u < WT; ++u) acc[u][g] = mfma_f16(ring[(hs + q) * WT + u], av[AP ? q & 1 : 0][g], acc[u][g]);
+      }
+#pragma unroll
+      for (int u = 0; u < WT; ++u) ring[(hs + q) * WT + u] = issue(u);
+      if (q == (WKS > 1 ? 1 : 0)) {
+        place_chunk(off2, h & 1 ? st1 : st0);
+        load_chunk(min(c + 4, nchunk - 1), h & 1 ? st1 : st0);
+      }
+      // left free, the scheduler hoists every read of the chunk ahead of the multiplies and runs
+      // out of registers
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();
+    const int o = off0;
+    off0 = off1; off1 = off2; off2 = o;
+  };
+  int c0 = 0;
+  for (; c0 + CYC <= nchunk; c0 += CYC) unrolled<0, CYC>([&](auto h) __attribute__((always_inline)) { chunk(c0 + h, h); });
+  unrolled<0, CYC - 1>([&](auto h) __attribute__((always_inline)) { if (c0 + h < nchunk) chunk(c0 + h, h); });
+  // epilogue: row g * 16 + row, columns n .. n + 3
+#pragma unroll
+  for (int g = 0; g < NGW; ++g) {
+    const int r = (g0 + g) * 16 + row;
+    if (r >= S) break;
+#pragma unroll
+    for (int u = 0; u < WT; ++u) {
+      const int n = (t0 + u) * 16 + cbase;
+      const f32x4 v = acc[u][g];
+      if constexpr (EPI == E_PART) {
+        *(f32x4*)((float*)ex.out + ((size_t)kc * S + r) * a.N + n) = v;
+      } else if constexpr (EPI == E_PART16) {
+        const int hr = ex.hrows > 0 ? ex.hrows : S, hb = r / hr, rr = r - hb * hr;
+        h16* o = (h16*)ex.out + ((size_t)kc * (S / hr) + hb) * hr * a.N;
+        *(h16x4*)(o + (ex.pack ? frag_index(rr, n, hr) : (size_t)rr * a.N + n)) =
+            (h16x4){(h16)v[0], (h16)v[1], (h16)v[2], (h16)v[3]};
+      } else {
+        h16x4 w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float y = v[q] + (float)bias[u][q];
+          w[q] = EPI == E_BIAS16 ? (h16)y : (h16)gelu_erf(a.gelu_r16 ? r16(y) : y);
+        }
+        h16* o = (h16*)ex.out + (size_t)r * a.N + n;
+        if (EPI == E_BIAS16 && ex.nsplit > 0) {
+          const int part = n / ex.nsplit;
+          o = (h16*)ex.out + ((size_t)part * S + r) * ex.nsplit + (n - part * ex.nsplit);
+        }
+        *(h16x4*)o = w;
+      }
+    }
+  }
+}
+
+template <int EPI, int NG, int WV, int CH, int WT, int RS, int RC, bool GA, bool HALF>
+__global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
   int b = blockIdx.x;
   const int per_ex = a.ks * a.wg_per_kc;
   int e, kc, tg;
@@ -99,218 +292,97 @@ __global__ void __launch_bounds__(WV * 64) k_wide(WArgs a) {
     tg = b - kc * a.wg_per_kc;
   }
   const WEx& ex = a.ex[e];
-  const int S = ex.S;
-  const int ksteps = a.K / 32;
-  const int KCW = a.K / a.ks, nsteps = KCW / 32, nchunk = KCW / CH;
-  const int t0 = (tg * WV + wave) * WT;               // this wave's WT adjacent 16-column tiles
-  const int k0 = kc * KCW;
-  // staging of one chunk: vector idx = u * nt + thread, row idx / NVR, columns (idx % NVR) * 8 .. +7;
-  // indices past the rows re-read the last vector (every load unconditional, see Stage)
-  constexpr int NT = WV * 64;
-  constexpr int NVR = CH / 8;                         // 16-byte vectors per row of a chunk
-  constexpr int NSV = (NG * 16 * NVR + NT - 1) / NT;  // vectors per thread at the most rows
-  const int total = S * NVR;
-  // each staging slot's element offset in the operand, the same at every chunk (a gathered row's
-  // index is read once)
-  size_t soff[NSV];
-#pragma unroll
-  for (int u = 0; u < NSV; ++u) {
-    const int idx = min(u * NT + (int)threadIdx.x, total - 1);
-    const int i = idx / NVR, kk = (idx - i * NVR) * 8;
-    const size_t src = ex.ids ? (size_t)max(ex.ids[(size_t)i * ex.ids_stride], 0) : (size_t)i;
-    soff[u] = src * ex.lda + kk;
-  }
-  h16x8 st[NSV];
-  auto load_chunk = [&](int c) {
-    const h16* base = ex.a + k0 + c * CH;
-#pragma unroll
-    for (int u = 0; u < NSV; ++u) st[u] = *(const h16x8*)(base + soff[u]);
-  };
-  auto place_chunk = [&](h16* buf) {
-#pragma unroll
-    for (int u = 0; u < NSV; ++u) {
-      const int idx = min(u * NT + (int)threadIdx.x, total - 1);
-      const int i = idx / NVR, kk = (idx - i * NVR) * 8;
-      *(h16x8*)(buf + i * WLDA + kk) = st[u];
-    }
-  };
-  // the wave's fragments, k-step by k-step, the WT tiles of a k-step together; past the last
-  // k-step the pointers stay there, so the ring's surplus refills re-read lines just fetched
-  const h16x8* lw = ex.w + ((size_t)t0 * ksteps + (size_t)kc * nsteps) * 64 + lane;
-  const size_t tstride = (size_t)ksteps * 64;         // next tile, same k-step
-  int lleft = nsteps * WT;
-  auto issue = [&](int u) -> h16x8 {
-    const h16x8 v = __builtin_nontemporal_load(lw + u * tstride);
-    if (u == WT - 1) {
-      const bool adv = lleft > WT;
-      lw += adv ? 64 : 0;
-      lleft -= adv ? WT : 0;
-    }
-    return v;
-  };
-  const int col = lane & 15, rbase = 4 * (lane >> 4);
-  float bias[WT] = {};
-  if constexpr (EPI == E_BIAS16 || EPI == E_GELU16) {
-#pragma unroll
-    for (int u = 0; u < WT; ++u) bias[u] = (float)ex.bias[(t0 + u) * 16 + col];
-  }
-  // operand chunk 0 first, then the weight prefetch (independent of it), then LDS
-  load_chunk(0);
-  __builtin_amdgcn_sched_barrier(0);
-  h16x8 ring[WSPF];
-#pragma unroll
-  for (int p = 0; p < WSPF; ++p) {
-    ring[p] = issue(p % WT);
-    // issued in slot order: each multiply then waits for its own slot alone (with the order left
-    // free, slot 0 went out seventh and the first multiply waited for the whole ring)
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  h16* buf0 = lds;
-  h16* buf1 = lds + (size_t)S * WLDA;
-  place_chunk(buf0);
-  lds_barrier();
-  const int row = lane & 15, kg = lane >> 4;
-  f32x4 acc[WT][NG];
-#pragma unroll
-  for (int u = 0; u < WT; ++u)
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[u][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  // lanes of rows past S read row 0: their products land in output rows that are never stored
-  // (every row group is multiplied, which keeps the loop free of branches)
-  int roff[NG];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) roff[g] = (g * 16 + row < S ? g * 16 + row : 0) * WLDA + kg * 8;
-  const h16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  // WRC chunks per ring cycle: slot p holds tile p % WT of k-step (p / WT) % WKS of chunk
-  // c0 + p / (WT WKS)
-  for (int c0 = 0; c0 < nchunk; c0 += WRC) {
-#pragma unroll
-    for (int h = 0; h < WRC; ++h) {
-      const int c = c0 + h;
-      // past the last chunk (a count that is not a multiple of WRC) zero fragments multiply the last
-      // chunk's rows, which are finite (0 x NaN from a buffer never written would poison the sums);
-      // the loop keeps no branches
-      const h16* cur = (min(c, nchunk - 1) & 1) ? buf1 : buf0;
-      h16* nxt = (c & 1) ? buf0 : buf1;
-      load_chunk(min(c + 1, nchunk - 1));
-#pragma unroll
-      for (int q = 0; q < WKS; ++q) {
-        const int p0 = (h * WKS + q) * WT;
-        h16x8 bf[WT];
-#pragma unroll
-        for (int u = 0; u < WT; ++u) bf[u] = (WRC == 1 || c < nchunk) ? ring[p0 + u] : zero8;
-        // one k-step at a time: each row group's operand read once, multiplied by the WT fragments
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const h16x8 av = *(const h16x8*)(cur + roff[g] + q * 32);
-#pragma unroll
-          for (int u = 0; u < WT; ++u) acc[u][g] = mfma_f16(av, bf[u], acc[u][g]);
-        }
-#pragma unroll
-        for (int u = 0; u < WT; ++u) ring[p0 + u] = issue(u);
-        // left free, the scheduler hoists every read of the chunk ahead of the multiplies and runs
-        // out of registers
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // chunk c + 1 goes to the other buffer (nobody reads it: every wave finished chunk c - 1
-      // before the last barrier); one barrier orders the stores before chunk c + 1's reads
-      if (c + 1 < nchunk) place_chunk(nxt);
-      lds_barrier();
-    }
-  }
-  // epilogue: rows g * 16 + rbase + q of column (t0 + u) * 16 + col
-#pragma unroll
-  for (int u = 0; u < WT; ++u) {
-    const int n = (t0 + u) * 16 + col;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if (g * 16 >= S) continue;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = g * 16 + rbase + q;
-        if (r >= S) continue;
-        const float v = acc[u][g][q];
-        if constexpr (EPI == E_PART) {
-          ((float*)ex.out)[((size_t)kc * S + r) * a.N + n] = v;
-        } else if constexpr (EPI == E_PART16) {
-          const int hr = ex.hrows > 0 ? ex.hrows : S, hb = r / hr, rr = r - hb * hr;
-          h16* o = (h16*)ex.out + ((size_t)kc * (S / hr) + hb) * hr * a.N;
-          o[ex.pack ? frag_index(rr, n, hr) : (size_t)rr * a.N + n] = (h16)v;
-        } else if constexpr (EPI == E_BIAS16) {
-          if (ex.nsplit > 0) {
-            const int part = n / ex.nsplit, nn = n - part * ex.nsplit;
-            ((h16*)ex.out)[((size_t)part * S + r) * ex.nsplit + nn] = (h16)(v + bias[u]);
-          } else {
-            ((h16*)ex.out)[(size_t)r * a.N + n] = (h16)(v + bias[u]);
-          }
-        } else {
-          const float w = v + bias[u];
-          ((h16*)ex.out)[(size_t)r * a.N + n] = (h16)gelu_erf(a.gelu_r16 ? r16(w) : w);
-        }
-      }
-    }
-  }
+  // an entry with at most half the rows (the first chunk expert) multiplies half the row groups
+  if (HALF && ex.S <= NG * 8) wide_unit<EPI, NG / 2, WV, CH, WT, RS, RC, GA>(a, ex, kc, tg);
+  else wide_unit<EPI, NG, WV, CH, WT, RS, RC, GA>(a, ex, kc, tg);
 }
 
-size_t wide_lds(int S_max, int ch) { return (size_t)2 * S_max * (ch + 8) * 2; }
-
-template <int EPI, int NG, int WV, int CH>
-int launch_wide_k(const WArgs& a, size_t lds, hipStream_t st) {
+template <int EPI, int NG, int WV, int CH, int WT, int RS, int RC, bool GA, bool HALF>
+int launch_wide_k(const WArgs& a, hipStream_t st) {
+  constexpr size_t lds = (size_t)3 * wide_rows(NG, WV, CH) * (CH + 8) * 2;
+  static_assert(lds <= 150 * 1024, "three chunk buffers fit the LDS");
   static unsigned long long attr_set = 0;
   int dev = 0;
   CFH_HIP(hipGetDevice(&dev));
   if (dev < 64 && !(attr_set & (1ull << dev))) {
-    CFH_HIP(hipFuncSetAttribute((const void*)k_wide<EPI, NG, WV, CH>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    CFH_HIP(hipFuncSetAttribute((const void*)k_wide<EPI, NG, WV, CH, WT, RS, RC, GA, HALF>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 150 * 1024));
     attr_set |= 1ull << dev;
   }
   const long long wgs = (long long)a.nex * a.ks * a.wg_per_kc;
-  hipLaunchKernelGGL((k_wide<EPI, NG, WV, CH>), dim3((unsigned)wgs), dim3(WV * 64), lds, st, a);
+  hipLaunchKernelGGL((k_wide<EPI, NG, WV, CH, WT, RS, RC, GA, HALF>), dim3((unsigned)wgs), dim3(WV * 64), lds, st, a);
   CFH_LAUNCH_CHECK();
   return CFH_OK;
 }
 
-// Shape checks of a wide launch (also used by the plan): CFH_OK when every unit of wv waves covers
-// whole tiles, every k-split a whole number of chunks, and the rows fit.
-int wide_check(const WArgs& a, int wv, int S_max, int ch = WCH) {
+// Shape of a wide launch's workgroups: wv waves, wv / rs of them side by side on wt adjacent 16-column
+// tiles each, every rs-th part of the rows.
+struct WShape {
+  int wv, wt, rs;
+  int tiles() const { return wv / rs * wt; }
+};
+constexpr WShape WSHAPES[] = {{4, 1, 2}, {4, 1, 1}, {4, 2, 1}, {4, 3, 1}, {8, 2, 1}, {8, 3, 1}};
+
+// 128-column chunks of fragments a wave keeps in flight.  The loads in flight are not what bounds these
+// launches: four chunks at {4, 2, 1} were 7% slower than one over a 13-request d = 2560 flow (each
+// workgroup's start and end carry the surplus), two at {8, 3, 1} do not fit the registers.
+constexpr int wide_rc(int wv, int wt) { return wv * wt == 8 || wv * wt == 24 ? 1 : 2; }
+
+// Shape checks of a wide launch (also used by the plan): CFH_OK when every workgroup covers whole
+// units, every k-split a whole number of chunks, and the rows fit.
+int wide_check(const WArgs& a, WShape s, int S_max, int ch = WCH) {
   if (a.nex < 1 || a.nex > 4 || a.N <= 0 || a.N % 16 || a.ks <= 0 || a.K % a.ks || (a.K / a.ks) % ch)
     return CFH_E_UNSUPPORTED;
-  if ((wv != 4 && wv != 6 && wv != 8 && wv != 12) || (a.N / 16) % (WT * wv) || S_max < 1 || S_max > WMAXR ||
-      wide_lds(S_max, ch) > 150 * 1024)
+  bool known = false;
+  for (const WShape& w : WSHAPES) known = known || (w.wv == s.wv && w.wt == s.wt && w.rs == s.rs);
+  if (!known || (a.N / 16) % s.tiles() || S_max < 1 || S_max > WMAXR)
     return CFH_E_UNSUPPORTED;
   if (a.pair && a.nex % 2) return CFH_E_UNSUPPORTED;
   return CFH_OK;
 }
 
-// Waves per workgroup of a wide launch over `units` units of `tiles` column tiles: the count
-// (WT tiles a wave, dividing tiles) that loads the busiest CU least -- rounds of 256 workgroups
-// times waves a workgroup -- preferring fewer waves a workgroup on ties.
-int wide_wv(int tiles, int units) {
+// Shape of a full-K launch of `units` units of `tiles` column tiles: the one with the least rounds of
+// 256 workgroups x (tiles a workgroup + 4), the 4 for what a workgroup costs whatever its tiles (its
+// start, the staging of the rows); the last listed on ties.
+WShape wide_shape_for(int tiles, int units) {
   constexpr int CUS = 256;
-  int best = 0;
+  WShape best = {};
   long long best_load = 0;
-  for (int wv : {4, 6, 8, 12}) {
-    if (tiles % (WT * wv)) continue;
-    const long long wgs = (long long)units * tiles / (WT * wv);
-    const long long load = (wgs + CUS - 1) / CUS * wv;
-    if (!best || load < best_load) {
-      best = wv;
+  for (const WShape& s : WSHAPES) {
+    if (tiles % s.tiles()) continue;
+    const long long wgs = (long long)units * tiles / s.tiles();
+    const long long load = (wgs + CUS - 1) / CUS * (s.tiles() + 4);
+    if (!best.wv || load <= best_load) {
+      best = s;
       best_load = load;
     }
   }
   return best;
 }
 
+// k-splits of a split-K launch: the most workgroups up to one a CU.
+int wide_ks(int N, int K, int units, WShape s) {
+  constexpr int CUS = 256;
+  int best = 0;
+  for (int ks = 1; ks <= K / WCH; ++ks) {
+    if (K % ks || (K / ks) % WCH) continue;
+    if (best && (long long)units * (N / 16 / s.tiles()) * ks > CUS) break;
+    best = ks;
+  }
+  return best;
+}
 
-template <int EPI, int CH = WCH>
-int launch_wide(const WArgs& a0, int wv, hipStream_t st) {
+// GA: the operand rows are gathered by WEx::ids.  HALVES: entries of at most half the largest one's
+// row groups multiply half as many (the flow's chunk experts).
+template <int EPI, bool HALVES = false, int CH = WCH, bool GA = false>
+int launch_wide(const WArgs& a0, WShape s, hipStream_t st) {
   WArgs a = a0;
   int S_max = 0;
   for (int e = 0; e < a.nex; ++e) S_max = std::max(S_max, a.ex[e].S);
-  if (wide_check(a, wv, S_max, CH)) return CFH_E_UNSUPPORTED;
+  if (wide_check(a, s, S_max, CH)) return CFH_E_UNSUPPORTED;
   for (int e = 0; e < a.nex; ++e)
-    if (a.ex[e].S < 1 || a.ex[e].lda < a.K || !a.ex[e].w || !a.ex[e].a || !a.ex[e].out) return CFH_E_INVALID;
-  a.wg_per_kc = (a.N / 16) / (WT * wv);
+    if (a.ex[e].S < 1 || a.ex[e].lda < a.K || !a.ex[e].w || !a.ex[e].a || !a.ex[e].out || !a.ex[e].ids == GA) return CFH_E_INVALID;
+  a.wg_per_kc = (a.N / 16) / s.tiles();
   // the side-by-side order needs a whole number of 8-workgroup runs per half (narrow widths such as
   // d = 640 have 5 a k-split: their paired launches keep the plain order, still one launch for both)
   const bool pair_runs = a.pair && ((long long)(a.nex / 2) * a.ks * a.wg_per_kc) % 8 == 0;
@@ -318,27 +390,23 @@ int launch_wide(const WArgs& a0, int wv, hipStream_t st) {
     a.map = MAP_XCD;
   else
     a.map = pair_runs ? MAP_PAIR : MAP_PLAIN;
-  const size_t lds = wide_lds(S_max, CH);
   const int ng = (S_max + 15) / 16;
-  // (the factor launches come in 4-wave workgroups only)
-  if constexpr (EPI == E_PART16) {
-    if (wv != 4) return CFH_E_UNSUPPORTED;
-    if (ng <= 2) return launch_wide_k<EPI, 2, 4, CH>(a, lds, st);
-    if (ng <= 4) return launch_wide_k<EPI, 4, 4, CH>(a, lds, st);
-    return launch_wide_k<EPI, 8, 4, CH>(a, lds, st);
-  } else {
-#define CFH_WIDE(G)                                                                 \
-  if (ng <= G) {                                                                    \
-    switch (wv) {                                                                   \
-      case 4: return launch_wide_k<EPI, G, 4, CH>(a, lds, st);                          \
-      case 6: return launch_wide_k<EPI, G, 6, CH>(a, lds, st);                          \
-      case 8: return launch_wide_k<EPI, G, 8, CH>(a, lds, st);                          \
-      default: return launch_wide_k<EPI, G, 12, CH>(a, lds, st);                        \
-    }                                                                               \
+  [[maybe_unused]] bool half = false;
+  for (int e = 0; e < a.nex; ++e) half = half || a.ex[e].S <= (ng <= 2 ? 0 : ng <= 4 ? 32 : 64);
+#define CFH_WIDE_S(G, W, T, R)                                                                                       \
+  if (ng <= G && s.wv == W && s.wt == T && s.rs == R) {                                                                        \
+    if constexpr (G > 2 && HALVES)                                                                                \
+      if (half) return launch_wide_k<EPI, G, W, CH, T, R, wide_rc(W, T), GA, true>(a, st);                           \
+    return launch_wide_k<EPI, G, W, CH, T, R, wide_rc(W, T), GA, false>(a, st);                                      \
   }
-  CFH_WIDE(2) CFH_WIDE(4) CFH_WIDE(8)
+#define CFH_WIDE(W, T, R) CFH_WIDE_S(2, W, T, R) CFH_WIDE_S(4, W, T, R) CFH_WIDE_S(8, W, T, R)
+  CFH_WIDE(4, 2, 1)
+  // (the factor launches and the gathered ones come in one shape only)
+  if constexpr (EPI != E_PART16 && !GA) {
+    CFH_WIDE(4, 1, 2) CFH_WIDE(4, 1, 1) CFH_WIDE(4, 3, 1) CFH_WIDE(8, 2, 1) CFH_WIDE(8, 3, 1)
+  }
 #undef CFH_WIDE
-  }
+#undef CFH_WIDE_S
   return CFH_E_UNSUPPORTED;
 }
 

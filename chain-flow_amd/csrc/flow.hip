@@ -762,8 +762,8 @@ int launch_xblock(const XblkArgs& a, hipStream_t st) {
 // Launch shapes of the wide kernels with `groups` request groups a launch.
 struct WideShape {
   int groups;
-  int wv_qkv, wv_w1, wv_kv, wv_qc; // full-K launches: waves per workgroup (wv_qc: unfolded cross q)
-  int wv_split;                    // split-K launches: waves per workgroup
+  WShape qkv, w1, kv, qc;          // full-K launches: workgroup shapes (qc: unfolded cross q)
+  WShape split;                    // split-K launches: workgroup shape
   int ks_wo, ks_ww2, ks_wout, ks_oc;  //                and k-splits (ks_oc: unfolded cross out-proj)
   bool ok;
 };
@@ -791,28 +791,6 @@ struct Plan {
   bool ok;
 };
 
-// Waves per workgroup of a wide launch whose workgroups should all be resident at once: the most
-// workgroups up to one per CU, then the most waves.  Two request groups of one expert then stream
-// each weight fragment side by side (on one XCD, `WArgs::pair`), and the second read hits the L2:
-// W1 at d = 4096 for two 16-request groups took 96.7 us a launch as 256 workgroups of 12 waves
-// (one group alone: 79.5 us), 127-135 us as 512 of 6 or 768 of 4, 159 us when the groups' reads
-// did not coincide.
-int wide_wv_resident(int tiles, int units) {
-  constexpr int CUS = 256;
-  int best = 0;
-  long long best_wgs = 0;
-  for (int wv : {4, 6, 8, 12}) {
-    if (tiles % (WT * wv)) continue;
-    const long long wgs = (long long)units * tiles / (WT * wv);
-    if (wgs > CUS) continue;
-    if (!best || wgs > best_wgs || (wgs == best_wgs && wv > best)) {
-      best = wv;
-      best_wgs = wgs;
-    }
-  }
-  return best ? best : wide_wv(tiles, units);
-}
-
 // Staging chunk of the wide factor launches: the widest that divides a head.
 int fold_chunk(int hd) {
   for (int ch : {128, 64, 32})
@@ -823,9 +801,9 @@ int fold_chunk(int hd) {
 // The factor launch with its staging chunk.
 int launch_wide_fold(const WArgs& a, int ch, hipStream_t st) {
   switch (ch) {
-    case 128: return launch_wide<E_PART16, 128>(a, 4, st);
-    case 64: return launch_wide<E_PART16, 64>(a, 4, st);
-    case 32: return launch_wide<E_PART16, 32>(a, 4, st);
+    case 128: return launch_wide<E_PART16, false, 128>(a, WShape{4, 2, 1}, st);
+    case 64: return launch_wide<E_PART16, false, 64>(a, WShape{4, 2, 1}, st);
+    case 32: return launch_wide<E_PART16, false, 32>(a, WShape{4, 2, 1}, st);
     default: return CFH_E_UNSUPPORTED;
   }
 }
@@ -837,28 +815,18 @@ WideShape wide_shape(const Plan& p, int groups) {
   s.groups = groups;
   const int units = groups * p.nch;
   if (units > 4) return s;
-  constexpr int CUS = 256;
   // split-K launches: 4-wave workgroups for one group; for two, 8-wave ones at one workgroup per CU,
   // so that the two groups' workgroups of a unit run together (d = 4096, 16 + 16 requests, E = 2:
   // 8.34 against 8.90 ms a flow pass with 4-wave workgroups)
-  s.wv_split = groups > 1 && (p.d / 16) % (WT * 8) == 0 ? 8 : 4;
-  auto ks_split = [&](int N, int K) {
-    int best = 0;
-    for (int ks = 1; ks <= K / WCH; ++ks) {
-      if (K % ks || (K / ks) % WCH) continue;
-      best = ks;
-      if ((long long)units * (N / 16 / (WT * s.wv_split)) * ks >= CUS) break;
-    }
-    return best;
-  };
-  auto wv_full = [&](int N) { return groups > 1 ? wide_wv_resident(N / 16, units) : wide_wv(N / 16, units); };
-  s.wv_qkv = wv_full(3 * p.d);
-  s.wv_w1 = wv_full(p.fd);
-  s.wv_kv = wide_wv(2 * p.d / 16, std::min(4, groups * std::min(4 / groups, p.nch * p.NL)));
+  s.split = groups > 1 && (p.d / 16) % 16 == 0 ? WShape{8, 2, 1} : WShape{4, 2, 1};
+  auto ks_split = [&](int N, int K) { return wide_ks(N, K, units, s.split); };
+  s.qkv = wide_shape_for(3 * p.d / 16, units);
+  s.w1 = wide_shape_for(p.fd / 16, units);
+  s.kv = wide_shape_for(2 * p.d / 16, std::min(4, groups * std::min(4 / groups, p.nch * p.NL)));
   s.ks_wo = ks_split(p.d, p.d);
   s.ks_ww2 = ks_split(p.d, p.fd);
   s.ks_wout = ks_split(p.d, p.d);
-  s.wv_qc = p.fold ? 0 : wv_full(p.d);
+  s.qc = p.fold ? WShape{} : wide_shape_for(p.d / 16, units);
   s.ks_oc = p.fold ? 0 : ks_split(p.d, p.d);
   auto wa = [&](int N, int K, int ks, int nex) {
     WArgs a = {};
@@ -867,15 +835,15 @@ WideShape wide_shape(const Plan& p, int groups) {
   };
   const int kv_nex = groups * std::min(4 / groups, p.nch * p.NL);
   s.ok = s.ks_wo > 0 && s.ks_ww2 > 0 && s.ks_wout > 0 &&
-         !wide_check(wa(3 * p.d, p.d, 1, units), s.wv_qkv, p.Smax) &&
-         !wide_check(wa(p.fd, p.d, 1, units), s.wv_w1, p.Smax) &&
-         !wide_check(wa(2 * p.d, p.d, 1, kv_nex), s.wv_kv, p.Ct) &&
-         !wide_check(wa(p.d, p.d, s.ks_wo, units), s.wv_split, p.Smax) &&
-         !wide_check(wa(p.d, p.fd, s.ks_ww2, units), s.wv_split, p.Smax) &&
-         !wide_check(wa(p.d, p.d, s.ks_wout, units), s.wv_split, p.Smax) &&
-         (p.fold ? !wide_check(wa(p.d, p.d, p.H, groups * p.nch), 4, p.Ct, p.fold_ch)
-                 : s.ks_oc > 0 && !wide_check(wa(p.d, p.d, 1, units), s.wv_qc, p.Smax) &&
-                       !wide_check(wa(p.d, p.d, s.ks_oc, units), s.wv_split, p.Smax));
+         !wide_check(wa(3 * p.d, p.d, 1, units), s.qkv, p.Smax) &&
+         !wide_check(wa(p.fd, p.d, 1, units), s.w1, p.Smax) &&
+         !wide_check(wa(2 * p.d, p.d, 1, kv_nex), s.kv, p.Ct) &&
+         !wide_check(wa(p.d, p.d, s.ks_wo, units), s.split, p.Smax) &&
+         !wide_check(wa(p.d, p.fd, s.ks_ww2, units), s.split, p.Smax) &&
+         !wide_check(wa(p.d, p.d, s.ks_wout, units), s.split, p.Smax) &&
+         (p.fold ? !wide_check(wa(p.d, p.d, p.H, groups * p.nch), WShape{4, 2, 1}, p.Ct, p.fold_ch)
+                 : s.ks_oc > 0 && !wide_check(wa(p.d, p.d, 1, units), s.qc, p.Smax) &&
+                       !wide_check(wa(p.d, p.d, s.ks_oc, units), s.split, p.Smax));
   return s;
 }
 
@@ -1285,7 +1253,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.qkv); x.a = gr[g].w.abuf[c]; x.lda = d;
         x.bias = (const h16*)PTR(c, B + L.qkv_b); x.out = gr[g].w.qkv[c]; x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_BIAS16>(a, sh.wv_qkv, st))) return rc;
+    if ((rc = launch_wide<E_BIAS16, true>(a, sh.qkv, st))) return rc;
   }
   // causal self attention of every (request, head), into the LN rows' buffer (free until the residual)
   {
@@ -1309,7 +1277,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.o); x.a = gr[g].w.abuf[c]; x.lda = d; x.out = gr[g].w.P[c];
         x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_PART>(a, sh.wv_split, st))) return rc;
+    if ((rc = launch_wide<E_PART, true>(a, sh.split, st))) return rc;
   }
   ResArgs r = {};
   r.nex = nex; r.d = d; r.mode = p.res_mode;
@@ -1343,7 +1311,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.qc); x.a = gr[g].w.abuf[c]; x.lda = d;
         x.bias = (const h16*)PTR(c, B + L.qc_b); x.out = gr[g].w.qkv[c]; x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_BIAS16>(a, sh.wv_qc, st))) return rc;
+    if ((rc = launch_wide<E_BIAS16, true>(a, sh.qc, st))) return rc;
     CrossArgs ca = {};
     ca.nex = nex; ca.H = p.H; ca.d = d; ca.hd = p.hd; ca.C = p.C;
     for (int g = 0; g < ng; ++g) {
@@ -1363,7 +1331,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.oc); x.a = gr[g].w.abuf[c]; x.lda = d; x.out = gr[g].w.P[c];
         x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_PART>(o, sh.wv_split, st))) return rc;
+    if ((rc = launch_wide<E_PART, true>(o, sh.split, st))) return rc;
   } else {
     // folded cross attention, two requests a subgroup
     XattArgs x = {};
@@ -1398,7 +1366,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.w1); x.a = gr[g].w.abuf[c]; x.lda = d;
         x.bias = (const h16*)PTR(c, B + L.w1_b); x.out = gr[g].w.g[c]; x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_GELU16>(a, sh.wv_w1, st))) return rc;
+    if ((rc = launch_wide<E_GELU16, true>(a, sh.w1, st))) return rc;
   }
   // W2: split-K partials
   {
@@ -1409,7 +1377,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
         x.w = (const h16x8*)PTR(c, B + L.w2); x.a = gr[g].w.g[c]; x.lda = fd; x.out = gr[g].w.P[c];
         x.S = S_of(g, c);
       }
-    if ((rc = launch_wide<E_PART>(a, sh.wv_split, st))) return rc;
+    if ((rc = launch_wide<E_PART, true>(a, sh.split, st))) return rc;
   }
   // residual + LayerNorm of the next block (out_norm after the last block)
   r.ks = sh.ks_ww2;
@@ -1457,7 +1425,7 @@ int per_draft_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout& 
         x.bias = (const h16*)PTR(c, BLK(l) + L.kv_b); x.out = gr[g].w.kvc[c] + (size_t)l * 2 * Cg * d; x.S = Cg;
         x.nsplit = d;
       }
-    if ((rc = launch_wide<E_BIAS16>(a, sh.wv_kv, st))) return rc;
+    if ((rc = launch_wide<E_BIAS16>(a, sh.kv, st))) return rc;
   }
   if (!p.fold) return CFH_OK;   // (the unfolded cross attention needs only the K/V rows)
   for (int g = 0; g < ng; ++g) {
@@ -1707,7 +1675,7 @@ int integrate_wide(const Plan& p, const cfh_flow_dims* dm, const cfh::ExpertLayo
           x.w = (const h16x8*)PTR(c, L.out); x.a = gr[g].w.abuf[c]; x.lda = d; x.out = gr[g].w.P[c];
           x.S = gr[g].Rg * (c + 1) * CS;
         }
-      if ((rc = launch_wide<E_PART>(a, sh.wv_split, st))) return rc;
+      if ((rc = launch_wide<E_PART, true>(a, sh.split, st))) return rc;
       for (int g = 0; g < ng; ++g)
         if ((rc = rows(gr[g], s, sh.ks_wout))) return rc;
     }

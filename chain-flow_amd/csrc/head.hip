@@ -1137,35 +1137,28 @@ PathPlan path_plan(int M, int d, int ffn, int order) {
 // gathered by the ancestor ids), split-K partials; k_path_sum; up: k_wide with the GELU epilogue
 // (fp16 rounding before the GELU, as torch's Linear then GELU modules); down: split-K partials;
 // k_path_out.
+constexpr WShape PATH_SPLIT = {4, 2, 1};   // workgroup shape of the split-K launches
+
 struct PathWide {
   bool ok;
-  int o_ks, dn_ks, up_wv;
+  int o_ks, dn_ks;
+  WShape up;
   size_t off_P, off_a, off_g, off_dn, total;
 };
 
 PathWide path_wide_plan(int M, int d, int ffn, int order) {
   PathWide p = {};
   const int pf = ffn * d;
-  constexpr int CUS = 256, WV = 4;
-  auto ks_for = [&](int units, int N, int K) {
-    int best = 0;
-    for (int ks = 1; ks <= K / WCH; ++ks) {
-      if (K % ks || (K / ks) % WCH) continue;
-      best = ks;
-      if ((long long)units * (N / 16 / (WT * WV)) * ks >= CUS) break;
-    }
-    return best;
-  };
-  p.o_ks = ks_for(order, d, d);
-  p.dn_ks = ks_for(1, d, pf);
-  p.up_wv = wide_wv(pf / 16, 1);
+  p.o_ks = wide_ks(d, d, order, PATH_SPLIT);
+  p.dn_ks = wide_ks(d, pf, 1, PATH_SPLIT);
+  p.up = wide_shape_for(pf / 16, 1);
   auto wa = [&](int nex, int N, int K, int ks) {
     WArgs a = {};
     a.nex = nex; a.N = N; a.K = K; a.ks = ks;
     return a;
   };
-  p.ok = order <= 4 && p.o_ks > 0 && p.dn_ks > 0 && p.up_wv > 0 && !wide_check(wa(order, d, d, p.o_ks), WV, M) &&
-         !wide_check(wa(1, pf, d, 1), p.up_wv, M) && !wide_check(wa(1, d, pf, p.dn_ks), WV, M);
+  p.ok = order <= 4 && p.o_ks > 0 && p.dn_ks > 0 && p.up.wv > 0 && !wide_check(wa(order, d, d, p.o_ks), PATH_SPLIT, M) &&
+         !wide_check(wa(1, pf, d, 1), p.up, M) && !wide_check(wa(1, d, pf, p.dn_ks), PATH_SPLIT, M);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -1623,7 +1616,7 @@ static int path_group_wide(const PathWide& pw, const void* const* ph, int order,
       x.w = (const h16x8*)ph[j]; x.a = (const h16*)embed_w; x.lda = d; x.ids = lastp + j; x.ids_stride = order;
       x.out = P + (size_t)j * pw.o_ks * M * d; x.S = M;
     }
-    if ((rc = launch_wide<E_PART>(a, 4, st))) return rc;
+    if ((rc = launch_wide<E_PART, false, WCH, true>(a, PATH_SPLIT, st))) return rc;
   }
   PathSumArgs ps = {};
   ps.P = P; ps.lastp = lastp; ps.g = (const h16*)ph[2 * order]; ps.b = (const h16*)ph[2 * order + 1]; ps.a = A;
@@ -1636,13 +1629,13 @@ static int path_group_wide(const PathWide& pw, const void* const* ph, int order,
     a.nex = 1; a.N = pf; a.K = d; a.ks = 1; a.gelu_r16 = 1;
     a.ex[0].w = (const h16x8*)ph[2 * order + 2]; a.ex[0].a = A; a.ex[0].lda = d;
     a.ex[0].bias = (const h16*)ph[2 * order + 3]; a.ex[0].out = G; a.ex[0].S = M;
-    if ((rc = launch_wide<E_GELU16>(a, pw.up_wv, st))) return rc;
+    if ((rc = launch_wide<E_GELU16>(a, pw.up, st))) return rc;
   }
   {
     WArgs a = {};
     a.nex = 1; a.N = d; a.K = pf; a.ks = pw.dn_ks;
     a.ex[0].w = (const h16x8*)ph[2 * order + 4]; a.ex[0].a = G; a.ex[0].lda = pf; a.ex[0].out = Pdn; a.ex[0].S = M;
-    if ((rc = launch_wide<E_PART>(a, 4, st))) return rc;
+    if ((rc = launch_wide<E_PART>(a, PATH_SPLIT, st))) return rc;
   }
   PathOutArgs po = {};
   po.P = Pdn; po.bias = (const h16*)ph[2 * order + 5]; po.pred = (const h16*)pred; po.hsum = (h16*)hsum;

@@ -262,8 +262,11 @@ int run_half(const VaePlan& p, const HalfPlan& hp, const HalfLayout& L, const ch
 // wide kernels (cfh_wide.h), so that a batch of sequences streams every weight once per group
 // instead of once per sequence.  Same launches and rounding points as the per-sequence form; the
 // self attention runs per (sequence, head) without a mask, the position rows repeat per sequence.
+constexpr WShape VAE_SPLIT = {4, 2, 1};   // workgroup shape of the split-K launches
+
 struct WideHalf {
-  int ks_in, wv_qkv, ks_o, wv_w1, ks_w2, ks_out;
+  int ks_in, ks_o, ks_w2, ks_out;
+  WShape qkv, w1;
 };
 
 struct VaeWide {
@@ -281,16 +284,7 @@ VaeWide vae_wide_plan(const cfh_vae_dims* dm, int rows, int G) {
   p.pcols = std::max({I, dm->hidden, dm->latent});
   if (G < 2 || p.S > WMAXR || I % WCH || hd % 8 || (size_t)3 * rows * hd * 2 + (size_t)rows * rows * 4 > 64 * 1024)
     return p;
-  constexpr int CUS = 256, WVS = 4;
-  auto ks_split = [&](int N, int K) {
-    int best = 0;
-    for (int ks = 1; ks <= K / WCH; ++ks) {
-      if (K % ks || (K / ks) % WCH) continue;
-      best = ks;
-      if ((long long)(N / 16 / (WT * WVS)) * ks >= CUS) break;
-    }
-    return best;
-  };
+  auto ks_split = [&](int N, int K) { return wide_ks(N, K, 1, VAE_SPLIT); };
   auto wa = [&](int N, int K, int ks) {
     WArgs a = {};
     a.nex = 1; a.N = N; a.K = K; a.ks = ks;
@@ -300,15 +294,15 @@ VaeWide vae_wide_plan(const cfh_vae_dims* dm, int rows, int G) {
   p.pks = 1;
   auto half = [&](WideHalf& h, int kin, int nout) {
     h.ks_in = kin % WCH ? 0 : ks_split(I, kin);
-    h.wv_qkv = wide_wv(3 * I / 16, 1);
+    h.qkv = wide_shape_for(3 * I / 16, 1);
     h.ks_o = ks_split(I, I);
-    h.wv_w1 = wide_wv(F / 16, 1);
+    h.w1 = wide_shape_for(F / 16, 1);
     h.ks_w2 = ks_split(I, F);
     h.ks_out = ks_split(nout, I);
-    p.ok = p.ok && h.ks_in > 0 && h.ks_o > 0 && h.ks_w2 > 0 && h.ks_out > 0 && h.wv_qkv > 0 && h.wv_w1 > 0 &&
-           !wide_check(wa(I, kin, h.ks_in), WVS, p.S) && !wide_check(wa(3 * I, I, 1), h.wv_qkv, p.S) &&
-           !wide_check(wa(I, I, h.ks_o), WVS, p.S) && !wide_check(wa(F, I, 1), h.wv_w1, p.S) &&
-           !wide_check(wa(I, F, h.ks_w2), WVS, p.S) && !wide_check(wa(nout, I, h.ks_out), WVS, p.S);
+    p.ok = p.ok && h.ks_in > 0 && h.ks_o > 0 && h.ks_w2 > 0 && h.ks_out > 0 && h.qkv.wv > 0 && h.w1.wv > 0 &&
+           !wide_check(wa(I, kin, h.ks_in), VAE_SPLIT, p.S) && !wide_check(wa(3 * I, I, 1), h.qkv, p.S) &&
+           !wide_check(wa(I, I, h.ks_o), VAE_SPLIT, p.S) && !wide_check(wa(F, I, 1), h.w1, p.S) &&
+           !wide_check(wa(I, F, h.ks_w2), VAE_SPLIT, p.S) && !wide_check(wa(nout, I, h.ks_out), VAE_SPLIT, p.S);
     p.pks = std::max({p.pks, h.ks_in, h.ks_o, h.ks_w2, h.ks_out});
   };
   half(p.enc, dm->hidden, dm->latent);
@@ -335,12 +329,11 @@ int run_half_wide(const VaeWide& p, const WideHalf& hp, const HalfLayout& L, con
     x.ex[0].w = wt; x.ex[0].a = a; x.ex[0].lda = lda; x.ex[0].out = o; x.ex[0].bias = b; x.ex[0].S = S;
     return x;
   };
-  constexpr int WVS = 4;
   int rc;
   ResArgs r = {};
   r.nex = 1; r.d = I; r.x[0] = w.x; r.P[0] = w.P; r.a[0] = w.a; r.rows[0] = S;
   // IN + position rows (row i of the group is position i % rows of its sequence), norm1 of layer 0
-  if ((rc = launch_wide<E_PART>(one(I, Kin, hp.ks_in, M(L.in), in, Kin, w.P, nullptr), WVS, st))) return rc;
+  if ((rc = launch_wide<E_PART>(one(I, Kin, hp.ks_in, M(L.in), in, Kin, w.P, nullptr), VAE_SPLIT, st))) return rc;
   r.mode = RES_POS16; r.ks = hp.ks_in; r.bias[0] = V(L.in_b); r.pos[0] = V(L.pos); r.pos_period = rows;
   r.g[0] = V(L.blk0 + L.n1_w); r.b[0] = V(L.blk0 + L.n1_b);
   if ((rc = launch_res(r, st))) return rc;
@@ -348,21 +341,21 @@ int run_half_wide(const VaeWide& p, const WideHalf& hp, const HalfLayout& L, con
   r.pos_period = 0;
   for (int l = 0; l < dm->layers; ++l) {
     const size_t B = L.blk0 + (size_t)l * L.blkstride;
-    if ((rc = launch_wide<E_BIAS16>(one(3 * I, I, 1, M(B + L.qkv), w.a, I, w.qkv, V(B + L.qkv_b)), hp.wv_qkv, st)))
+    if ((rc = launch_wide<E_BIAS16>(one(3 * I, I, 1, M(B + L.qkv), w.a, I, w.qkv, V(B + L.qkv_b)), hp.qkv, st)))
       return rc;
     SelfArgs sa = {};
     sa.nex = 1; sa.R = G; sa.H = H; sa.d = I; sa.hd = I / H; sa.bidir = 1;
     sa.qkv[0] = w.qkv; sa.out[0] = w.a; sa.S[0] = S; sa.Sr[0] = rows;
     if ((rc = launch_self_attn(sa, st))) return rc;
-    if ((rc = launch_wide<E_PART>(one(I, I, hp.ks_o, M(B + L.o), w.a, I, w.P, nullptr), WVS, st))) return rc;
+    if ((rc = launch_wide<E_PART>(one(I, I, hp.ks_o, M(B + L.o), w.a, I, w.P, nullptr), VAE_SPLIT, st))) return rc;
     r.ks = hp.ks_o; r.bias[0] = V(B + L.o_b); r.g[0] = V(B + L.n2_w); r.b[0] = V(B + L.n2_b);
     if ((rc = launch_res(r, st))) return rc;
     {
       WArgs a = one(F, I, 1, M(B + L.w1), w.a, I, w.g, V(B + L.w1_b));
       a.gelu_r16 = 1;
-      if ((rc = launch_wide<E_GELU16>(a, hp.wv_w1, st))) return rc;
+      if ((rc = launch_wide<E_GELU16>(a, hp.w1, st))) return rc;
     }
-    if ((rc = launch_wide<E_PART>(one(I, F, hp.ks_w2, M(B + L.w2), w.g, F, w.P, nullptr), WVS, st))) return rc;
+    if ((rc = launch_wide<E_PART>(one(I, F, hp.ks_w2, M(B + L.w2), w.g, F, w.P, nullptr), VAE_SPLIT, st))) return rc;
     r.ks = hp.ks_w2; r.bias[0] = V(B + L.w2_b);
     if (l + 1 < dm->layers) {
       r.g[0] = V(B + L.blkstride + L.n1_w); r.b[0] = V(B + L.blkstride + L.n1_b);
@@ -371,7 +364,7 @@ int run_half_wide(const VaeWide& p, const WideHalf& hp, const HalfLayout& L, con
     }
     if ((rc = launch_res(r, st))) return rc;
   }
-  if ((rc = launch_wide<E_PART>(one(Nout, I, hp.ks_out, M(L.out), w.a, I, w.P, nullptr), WVS, st))) return rc;
+  if ((rc = launch_wide<E_PART>(one(Nout, I, hp.ks_out, M(L.out), w.a, I, w.P, nullptr), VAE_SPLIT, st))) return rc;
   ReduceArgs ra = {};
   ra.nex = 1; ra.nl = 1; ra.ks = hp.ks_out; ra.rows = S; ra.N = Nout; ra.d = Nout; ra.kv = 0;
   ra.P[0] = w.P; ra.b[0] = V(L.out_b); ra.out[0] = out;
