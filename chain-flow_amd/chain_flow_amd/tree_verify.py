@@ -87,7 +87,9 @@ def tree_attn_merge(query, key, value, output, prefix_out, prefix_lse, idx_pad, 
     pout = prefix_out.contiguous()
     plse = prefix_lse.to(torch.float32).contiguous()
     idx = _i32(idx_pad, dev)
-    mask = torch.as_tensor(not_anc).to(dev, torch.uint8).contiguous()
+    # (a bool mask's bytes are 0 and 1 already: reinterpreted, not converted by a launch)
+    mask = torch.as_tensor(not_anc).to(dev).contiguous()
+    mask = mask.view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8)
     _lib.check(_lib.lib().cfh_tree_attn_merge(
         query.data_ptr(), query.stride(0), key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0),
         output.data_ptr(), output.stride(0), pout.data_ptr(), plse.data_ptr(), idx.data_ptr(), mask.data_ptr(),

@@ -7,6 +7,8 @@
 //     (patch tree_greedy_descent_kernel / tree_rejection_sample, lines 433-550).
 #include <math.h>
 
+#include <type_traits>
+
 #include "cfh_kernels.h"
 
 namespace {
@@ -120,7 +122,7 @@ __device__ __forceinline__ void widen(const typename LaneVec<EPL>::type& r, floa
   for (int e = 0; e < EPL; ++e) o[e] = ld2<IS_BF16>(t, e);
 }
 
-constexpr int TA_BATCH = 8;   // key / value rows whose loads are in flight together
+constexpr int TA_BATCH = 8;   // key (or value) rows whose loads are in flight together past 16 columns
 
 // The unmasked columns of the row, lowest first, as two wave-uniform 64-bit sets.
 struct ColSet {
@@ -160,79 +162,97 @@ __global__ void __launch_bounds__(TA_WAVES * 64) k_tree_attn(AttnArgs a) {
   auto row_of = [&](int m) { return m < 64 ? __builtin_amdgcn_readlane(ix0, m) : __builtin_amdgcn_readlane(ix1, m - 64); };
   float qv[EPL];
   widen<IS_BF16, EPL>(qraw, qv);
-  // round trip 2 (per TA_BATCH columns): the key AND value rows of the unmasked columns together;
-  // the scores go to LDS (column ordinal order), then the max, the denominator and the weighted
-  // sum follow in increasing column order
+  // round trip 2: the key AND value rows of the unmasked columns together; then the scores, the max,
+  // the denominator and the weighted sum in increasing column order
   float mx = -INFINITY, den = 0.f;
   float acc[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
-  int ncol = 0;
-  while (!cs.empty()) {
-    int ms[TA_BATCH];
-    VT kr[TA_BATCH], vr[TA_BATCH];
-    int cnt = 0;
+  auto score = [&](const VT& kr) {   // the wave total is the same in every lane
+    float kv[EPL];
+    widen<IS_BF16, EPL>(kr, kv);
+    float part = 0.f;
 #pragma unroll
-    for (int c = 0; c < TA_BATCH; ++c) {
-      ms[c] = cs.empty() ? -1 : cs.pop();
-      if (ms[c] >= 0) ++cnt;
-      const size_t rr = (size_t)row_of(max(ms[c], 0));
+    for (int e = 0; e < EPL; ++e) part += qv[e] * kv[e];
+    return wave_sum(part) * a.scale;
+  };
+  auto add = [&](float p, const VT& vr) {
+    float vv[EPL];
+    widen<IS_BF16, EPL>(vr, vv);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[e] += p * vv[e];
+  };
+  // NB >= the row's columns: every row loaded once, the scores in registers
+  auto once = [&](auto nb_c, int cnt) {
+    constexpr int NB = decltype(nb_c)::value;
+    VT kr[NB], vr[NB];
+    float sm[NB];
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      const size_t rr = (size_t)row_of(cs.empty() ? 0 : cs.pop());   // (past the columns: never used)
       kr[c] = *(const VT*)(a.k + rr * a.k_ld + (size_t)hk * D + lane * EPL);
       vr[c] = *(const VT*)(a.v + rr * a.v_ld + (size_t)hk * D + lane * EPL);
     }
 #pragma unroll
-    for (int c = 0; c < TA_BATCH; ++c) {
-      if (c >= cnt) break;
-      float kv[EPL];
-      widen<IS_BF16, EPL>(kr[c], kv);
-      float part = 0.f;
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) part += qv[e] * kv[e];
-      // the wave total is the same in every lane: each lane stores it and later reads back its own
-      const float sm = wave_sum(part) * a.scale;
-      sc[wave][ncol + c] = sm;
-      mx = fmaxf(mx, sm);
+    for (int c = 0; c < NB; ++c) {
+      sm[c] = c < cnt ? score(kr[c]) : -INFINITY;
+      mx = fmaxf(mx, sm[c]);
     }
-    ncol += cnt;
-    // keep the value rows of this batch in registers for the weighted sum below only when every
-    // column fits one batch (the common tree: depth + 1 <= TA_BATCH ancestors)
-    if (cs.empty() && ncol == cnt) {
-      for (int c = 0; c < cnt; ++c) den += expf(sc[wave][c] - mx);
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < cnt) den += sm[c] = expf(sm[c] - mx);
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c < cnt) add(sm[c] / den, vr[c]);
+  };
+  // A row of up to 16 columns (a node's ancestors and itself) takes the least of 4, 8 and 16 that
+  // holds them.  Rows of more than 8 used to go through the two passes below, their value rows read
+  // twice: four 40-node trees of depth 10, 16 / 4 heads of 256: 11.6 -> 8.7 us.
+  const int ncols = __popcll(cs.lo) + __popcll(cs.hi);
+  if (ncols <= 4) {
+    once(std::integral_constant<int, 4>{}, ncols);
+  } else if (ncols <= 8) {
+    once(std::integral_constant<int, 8>{}, ncols);
+  } else if (ncols <= 16) {
+    once(std::integral_constant<int, 16>{}, ncols);
+  } else {
+    // batches of TA_BATCH columns: the scores to LDS (column ordinal order), then the denominator and
+    // a pass over the value rows
+    int ncol = 0;
+    while (!cs.empty()) {
+      VT kr[TA_BATCH];
+      int cnt = 0;
+#pragma unroll
+      for (int c = 0; c < TA_BATCH; ++c) {
+        const int m = cs.empty() ? -1 : cs.pop();
+        if (m >= 0) ++cnt;
+        kr[c] = *(const VT*)(a.k + (size_t)row_of(max(m, 0)) * a.k_ld + (size_t)hk * D + lane * EPL);
+      }
 #pragma unroll
       for (int c = 0; c < TA_BATCH; ++c) {
         if (c >= cnt) break;
-        const float p = expf(sc[wave][c] - mx) / den;
-        float vv[EPL];
-        widen<IS_BF16, EPL>(vr[c], vv);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] += p * vv[e];
+        const float sm = score(kr[c]);
+        sc[wave][ncol + c] = sm;   // each lane stores it and later reads back its own
+        mx = fmaxf(mx, sm);
       }
-      ncol = -1;   // done
+      ncol += cnt;
     }
-  }
-  if (ncol >= 0) {
-    // more than one batch of columns: the denominator, then a second pass over the value rows
     for (int c = 0; c < ncol; ++c) den += expf(sc[wave][c] - mx);
     ColSet cv = {__ballot(ok0), __ballot(ok1)};
     int c = 0;
     while (!cv.empty()) {
-      int ms[TA_BATCH];
       VT vr[TA_BATCH];
       int cnt = 0;
 #pragma unroll
       for (int u = 0; u < TA_BATCH; ++u) {
-        ms[u] = cv.empty() ? -1 : cv.pop();
-        if (ms[u] >= 0) ++cnt;
-        vr[u] = *(const VT*)(a.v + (size_t)row_of(max(ms[u], 0)) * a.v_ld + (size_t)hk * D + lane * EPL);
+        const int m = cv.empty() ? -1 : cv.pop();
+        if (m >= 0) ++cnt;
+        vr[u] = *(const VT*)(a.v + (size_t)row_of(max(m, 0)) * a.v_ld + (size_t)hk * D + lane * EPL);
       }
 #pragma unroll
       for (int u = 0; u < TA_BATCH; ++u) {
         if (u >= cnt) break;
-        const float p = expf(sc[wave][c + u] - mx) / den;
-        float vv[EPL];
-        widen<IS_BF16, EPL>(vr[u], vv);
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[e] += p * vv[e];
+        add(expf(sc[wave][c + u] - mx) / den, vr[u]);
       }
       c += cnt;
     }
@@ -263,6 +283,7 @@ __global__ void __launch_bounds__(TA_WAVES * 64) k_tree_attn(AttnArgs a) {
 // (value, first index), reduced over the wave and the workgroup (the larger value, then the lower
 // index) into ws[r][split]; the descent kernel then reduces a request's rows' slices in slice order.
 constexpr int ACC_SPLIT = 16;
+constexpr int ACC_LB = 8;    // 16-byte loads in flight a thread
 
 struct ArgPart { float v; int i; };
 
@@ -283,13 +304,21 @@ __global__ void __launch_bounds__(256) k_argmax_part(const u16* logits, int V, l
     // 8-element vectors over the aligned middle of [c0, c1), scalars at both ends
     const int v0 = (c0 + 7) / 8, v1 = c1 / 8;
     for (int j = c0 + threadIdx.x; j < min(c1, v0 * 8); j += blockDim.x) better(best, bix, ld2<IS_BF16>(row, j), j);
-    for (int u = v0 + threadIdx.x; u < v1; u += blockDim.x) {
-      const uint4 raw = *(const uint4*)(row + (size_t)u * 8);
-      const u16* t = (const u16*)&raw;
+    // ACC_LB vectors a thread in flight (one at a time: 16.5, so: 15.6 us for 164 rows x 248,320); past
+    // the slice the last vector again, which changes nothing
+    for (int u0 = v0 + threadIdx.x; u0 < v1; u0 += ACC_LB * 256) {
+      uint4 raw[ACC_LB];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = ld2<IS_BF16>(t, e);
-        if (v > best) { best = v; bix = u * 8 + e; }   // increasing index within a thread: > keeps the first
+      for (int b = 0; b < ACC_LB; ++b) raw[b] = *(const uint4*)(row + (size_t)min(u0 + b * 256, v1 - 1) * 8);
+#pragma unroll
+      for (int b = 0; b < ACC_LB; ++b) {
+        const int u = min(u0 + b * 256, v1 - 1);
+        const u16* t = (const u16*)&raw[b];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float v = ld2<IS_BF16>(t, e);
+          if (v > best) { best = v; bix = u * 8 + e; }   // increasing index within a thread: > keeps the first
+        }
       }
     }
     for (int j = max(v1 * 8, v0 * 8) + threadIdx.x; j < c1; j += blockDim.x) better(best, bix, ld2<IS_BF16>(row, j), j);
@@ -340,9 +369,13 @@ __global__ void __launch_bounds__(64) k_tree_descent(DescentArgs a) {
   const bool lds = n <= ACC_LDS;
   for (int j = threadIdx.x; j <= n; j += blockDim.x) {
     const ArgPart* p = a.ws + (size_t)(s0 + j) * ACC_SPLIT;
+    ArgPart q[ACC_SPLIT];
+#pragma unroll
+    for (int k = 0; k < ACC_SPLIT; ++k) q[k] = p[k];
     float bv = -INFINITY;
     int bi = a.V;
-    for (int k = 0; k < ACC_SPLIT; ++k) better(bv, bi, p[k].v, p[k].i);
+#pragma unroll
+    for (int k = 0; k < ACC_SPLIT; ++k) better(bv, bi, q[k].v, q[k].i);
     bi = bi < a.V ? bi : 0;
     a.row_argmax[s0 + j] = bi;
     if (lds) s_arg[j] = bi;

@@ -89,6 +89,37 @@ def test_tree_attn_merge_matches_oracle(cuda, dtype, S, N, H, Hkv, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 256), (torch.float16, 64)])
+def test_tree_attn_every_column_count_matches_oracle(cuda, dtype, D):
+    """One path of 21 nodes: rows of 1 to 21 columns, over the edges (4, 8, 16) of the forms a row takes
+    by its count; and node 20 with no column at all (its suffix half weighs nothing).  Bounds as in
+    test_tree_attn_merge_matches_oracle."""
+    S, N, H, Hkv = 1, 21, 4, 2
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(N, h, D, generator=g).to(dtype) for h in (H, Hkv, Hkv))
+    out, pout = (torch.randn(N, H, D, generator=g).to(dtype) for _ in range(2))
+    plse = (torch.randn(H, N, generator=g) + 3.0).float()
+    idx = np.arange(N).reshape(S, N)
+    not_anc = ~np.tril(np.ones((N, N), dtype=bool))[None]
+    not_anc[0, N - 1] = True
+    print(f"[tree attn columns] {dtype} D={D}", flush=True)
+    o_gpu = out.to(cuda)
+    tree_attn_merge(q.to(cuda), k.to(cuda), v.to(cuda), o_gpu, pout.to(cuda), plse.to(cuda), torch.as_tensor(idx),
+                    torch.as_tensor(not_anc).to(cuda), D ** -0.5)
+    torch.cuda.synchronize()
+    num = "bf16" if dtype == torch.bfloat16 else "fp16"
+    keep = slice(0, N - 1)
+    ref = otv.tree_suffix_merge(to64(q), to64(k), to64(v), to64(pout), to64(plse), idx, not_anc, D ** -0.5,
+                                numerics=num)[keep]
+    got = to64(o_gpu)[keep]
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    worst = float((np.abs(got - ref) / (np.abs(ref) * ulp + 1e-6)).max())
+    print(f"  rel err {rel_err(got, ref):.2e}, worst {worst:.2f} ulp", flush=True)
+    assert rel_err(got, ref) < 2e-3 and worst <= 2.0
+    assert torch.equal(o_gpu[N - 1].cpu(), pout[N - 1]) or torch.isnan(o_gpu[N - 1].float()).all()
+
+
+@pytest.mark.gpu
 def test_tree_greedy_accept_matches_oracle(cuda):
     rng = np.random.default_rng(5)
     V = 248320
