@@ -78,6 +78,7 @@ SIGNATURES = {
     "cfh_head_gemm_topk_packed": (_I, [_VP, _I, _I, _VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP]),
     "cfh_head_topk_grouped": (_I, [_VP, _I, _I, _I, _VP, _VP, C.c_longlong, _I, _VP, _VP, _I, _I, _VP, _I, _VP, _VP,
                                    _VP, _VP, _VP]),
+    "cfh_head_gemm16_markov_topk": (_I, [_VP, _I, _I, _VP, _I, _VP, _I, _VP, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP]),
     "cfh_head_gemm16_topk": (_I, [_VP, _I, _I, _VP, _I, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP]),
     "cfh_path_ws_bytes": (_I64, [_I, _I, _I, _I]),
     "cfh_path_residual": (_I, [C.POINTER(_VP), _I, _I, _I, _VP, _I, _I, _VP, _VP, C.c_longlong, _I, _VP, _VP,

@@ -18,6 +18,7 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
 
 GEMV_ROWS = 8        # rows the GEMV head takes per launch; more go through the MFMA GEMM head
 GEMM_ROWS = 256      # rows of one GEMM head launch
+GEMM_MARKOV_ROWS = 128   # ... with the markov bias computed in it
 
 
 class ShortlistHead:
@@ -133,13 +134,24 @@ class ShortlistHead:
 
     def gemm_topk(self, h: torch.Tensor, k: int, prev: torch.Tensor | None, logits: torch.Tensor | None, out):
         """``topk`` of up to 256 rows on the MFMA GEMM head (cfh_head_gemm16_topk) over the packed
-        image; with ``prev`` (one global id per row) the markov bias fp16(w1[prev] . w2_sl) first, as
-        logits of the image's markov rows, added before the head logits' last rounding."""
+        image; with ``prev`` (one global id per row) the markov bias fp16(w1[prev] . w2_sl) is added
+        before the head logits' last rounding: in the same launch for up to 128 rows
+        (cfh_head_gemm16_markov_topk), else first, as logits of the image's markov rows."""
         M = h.shape[0]
         L = _lib.lib()
         st = _lib.stream_handle()
         h = h.contiguous()
         bias = None
+        if prev is not None and self.w1 is not None and M <= GEMM_MARKOV_ROWS and self.r % 256 == 0:
+            ids32 = prev if prev.dtype == torch.int32 and prev.is_cuda and prev.stride(0) > 0 else \
+                prev.to(h.device, torch.int32).contiguous()
+            vals, ids, lse = out
+            ws = self.workspace(M, k, h.device)
+            _lib.check(L.cfh_head_gemm16_markov_topk(
+                h.data_ptr(), M, self.d, self.image.data_ptr(), self.n, self.w1.data_ptr(), self.w1.shape[0],
+                ids32.data_ptr(), ids32.stride(0), self.r, k, _lib.ptr(logits), vals.data_ptr(), ids.data_ptr(),
+                lse.data_ptr(), ws.data_ptr(), st), "cfh_head_gemm16_markov_topk")
+            return vals, ids, lse
         if prev is not None and self.w1 is not None:
             a = self.w1.index_select(0, prev.to(torch.long)).contiguous()          # [M, r]
             bias = torch.empty(M, self.n, dtype=torch.float16, device=h.device)

@@ -561,15 +561,23 @@ struct GemmArgs {
   uint16_t* logits;    // [M][n] bf16 (F16: fp16) or null
   void* ws;
   int M, d, n, k, nsets;   // k = 0: logits only, no top-k
+  // MK: the markov bias computed in the kernel: w2's image rows [n][r] (packed), w1 [V][r], the row's
+  // markov parent mids[row * mid_stride] (clamped to w1's rows), r % 256 == 0
+  const uint16_t* mw;
+  const uint16_t* ma;
+  const int* mids;
+  int mid_stride, r, V;
 };
 
 // The 16-bit logit of a GEMM accumulator: bf16(acc), or fp16(acc) -- fp16(fp16(acc) + bias) with a
 // bias, the rounding points of the GEMV head's fp16(fp16(h.W) + fp16(A.W2)).
-template <bool F16>
-__device__ __forceinline__ uint16_t gemm_logit(float acc, const uint16_t* bias) {
+// MK: the bias is mb.
+template <bool F16, bool MK>
+__device__ __forceinline__ uint16_t gemm_logit(float acc, const uint16_t* bias, h16 mb) {
   if constexpr (F16) {
     h16 v = (h16)acc;
-    if (bias) v = (h16)((float)v + (float)__builtin_bit_cast(h16, *bias));
+    if constexpr (MK) v = (h16)((float)v + (float)mb);
+    else if (bias) v = (h16)((float)v + (float)__builtin_bit_cast(h16, *bias));
     return __builtin_bit_cast(uint16_t, v);
   } else {
     return __builtin_bit_cast(uint16_t, (__bf16)acc);
@@ -593,9 +601,9 @@ __device__ __forceinline__ unsigned umed3(unsigned a, unsigned b, unsigned c) { 
 // columns l*CPL .. l*CPL+CPL-1 as 32-bit keys (order-preserving 16-bit logit << 16 | 0xFFFF -
 // column), so one integer max picks the larger logit and, on a tie, the lower column.  Key 0 = no
 // column.  The block's top-k and (max, sum of exp) go to the candidate lists for the merge.
-template <int MTW, int NT, int COLS, int NTHR, int ROWS, bool F16>
-__device__ __forceinline__ void gemm_finish(const GemmArgs& a, const f32x4 (&acc)[MTW][NT], uint16_t* lg, int rt0,
-                                            int c0) {
+template <int MTW, int NT, int COLS, int NTHR, int ROWS, bool F16, bool MK>
+__device__ __forceinline__ void gemm_finish(const GemmArgs& a, const f32x4 (&acc)[MTW][NT],
+                                            const h16* mb, uint16_t* lg, int rt0, int c0) {
   constexpr int LST = COLS + 8, CPL = COLS / 16;
   static_assert(CPL % 8 == 0, "a lane's columns are read as 16-byte vectors");
   const int lane = threadIdx.x & 63;
@@ -614,8 +622,10 @@ __device__ __forceinline__ void gemm_finish(const GemmArgs& a, const f32x4 (&acc
           const int r = (rt0 + mt) * 16 + 4 * g + q;
           const int c = c0 + t * 16 + col;
           const int j = blockIdx.x * COLS + c;
-          lg[r * LST + c] = gemm_logit<F16>(acc[mt][t][q],
-                                            bias ? a.bias + (size_t)min(r, a.M - 1) * a.n + min(j, a.n - 1) : nullptr);
+          lg[r * LST + c] =
+              gemm_logit<F16, MK>(acc[mt][t][q],
+                                  bias ? a.bias + (size_t)min(r, a.M - 1) * a.n + min(j, a.n - 1) : nullptr,
+                                  MK ? mb[r * LST + c] : (h16)0.f);
         }
     if (a.logits) {
 #pragma unroll
@@ -770,15 +780,30 @@ __device__ __forceinline__ void gemm_finish(const GemmArgs& a, const f32x4 (&acc
   }
 }
 
+template <int MT, int NT, int GW, int MS>
+constexpr size_t gemm_lds() {
+  const size_t xbuf = 2 * (size_t)MT * 16 * GKC * 2;                      // x double buffer
+  const size_t lgt = (size_t)MT * 16 * (GW / MS * NT * 16 + 8) * 2 +      // the block's logits,
+                     ((size_t)MT * 16 + 1) * (KMAX * 4 + 8);              // staged winners' keys, (max, sum)
+  return xbuf > lgt ? xbuf : lgt;
+}
+
 // MS: the MT row tiles are split over MS waves that share the same NT column tiles (the waves of a
 // workgroup are NG = GW / MS column groups times MS row groups), so each x operand read from LDS
 // feeds NT MFMAs and each wave keeps NT tiles of weight fragments in flight.
-template <int MT, int NT, int GW, bool PK, bool F16, int MS>
+//
+// MK: the markov bias first, as r / GKC more chunks before the head's: the same pipeline, its x rows
+// gathered from w1 and its fragments from w2's image; their sums, rounded to fp16, wait in LDS for the
+// epilogue (in registers, 49 spilled).  (As a launch of its own, with the gather, it wrote and read 16 MB of biases: 128
+// rows x 62,642, d = 4096, r = 256: 26 us and the gather's 9 us beside the head's 108 us, 102 us
+// fused.)
+template <int MT, int NT, int GW, bool PK, bool F16, int MS, bool MK>
 __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   // [2][MT*16][GKC], each row's 16-byte slots XOR-swizzled by the row's low 4 bits: the 16 rows
   // an MFMA operand read touches then fall on 16 different bank groups
   extern __shared__ __align__(16) uint16_t xs[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // (the wave index read as a scalar keeps the image's pointers out of the vector registers)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   constexpr int ROWS = MT * 16, NG = GW / MS, MTW = MT / MS;
   static_assert(NG * MS == GW && MTW * MS == MT, "the row tiles and waves must split evenly");
   const int ng = wave % NG, mh = wave / NG;
@@ -790,7 +815,7 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   for (int t = 0; t < NT; ++t) {
     if constexpr (PK) {
       const int tile = min(tile0 + t, (a.n + 15) / 16 - 1);
-      wp[t] = (const bf16x8*)a.W + (size_t)tile * (a.d / 32) * 64 + lane;
+      wp[t] = (const bf16x8*)a.W + (size_t)tile * (a.d / 32) * 64;
     } else {
       const int j = (tile0 + t) * 16 + (lane & 15);
       const int jc = j < a.n ? j : a.n - 1;
@@ -799,6 +824,20 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
     }
   }
   const int nchunks = a.d / GKC;
+  static_assert(!MK || (PK && F16), "the markov rows are those of a packed fp16 image");
+  const int nm = MK ? a.r / GKC : 0;                  // markov chunks, an even count
+  const bf16x8* wm[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    wm[t] = MK ? (const bf16x8*)a.mw + (size_t)min(tile0 + t, (a.n + 15) / 16 - 1) * (a.r / 32) * 64 : nullptr;
+  // the fragment pointers of chunk c, the markov chunks counted before the head's
+  auto wchunk = [&](int c, int t) {
+    return MK && c < nm ? wm[t] + c * GPF * KS : wp[t] + min(c - nm, nchunks - 1) * GPF * KS;
+  };
+  const unsigned loff = PK ? lane * 16 : 0;           // the lane's share of an image fragment
+  auto frag = [&](const bf16x8* w, int p) __attribute__((always_inline)) {
+    return wload<PK>((const bf16x8*)((const char*)(w + p * KS) + loff));
+  };
   // two register sets of weight fragments, for even and odd chunks: while chunk c is multiplied
   // from one set, the other holds chunk c+1 in flight, and each k-step's fragments are reloaded
   // with chunk c+2's right after their last multiply, in the same registers (nothing is copied at
@@ -808,14 +847,27 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   for (int p = 0; p < GPF; ++p)
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      bqa[p][t] = wload<PK>(wp[t] + p * KS);
-      bqb[p][t] = wload<PK>(wp[t] + (min(1, nchunks - 1) * GPF + p) * KS);
+      bqa[p][t] = frag(wchunk(0, t), p);
+      bqb[p][t] = frag(wchunk(1, t), p);
     }
   // x chunk: ROWS x 16 vectors of 8, XV a thread (vector idx = row*16 + v); branch-free, rows past
   // M repeat row M-1 (their products are never read), so the wait counts before the multiplies
   // count these loads exactly and leave the weight loads in flight
   constexpr int XV = ROWS * 16 / (GW * 64);
   static_assert(XV * GW * 64 == ROWS * 16, "x chunk must split evenly over the workgroup");
+  int mid[MK ? XV : 1];
+  if constexpr (MK) {
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const int row = min((int)(threadIdx.x + i * GW * 64) >> 4, a.M - 1);
+      mid[i] = min(max(a.mids[(size_t)row * a.mid_stride], 0), a.V - 1);
+    }
+  }
+  auto load_xm = [&](int c, bf16x8* xr) {             // markov chunk c
+#pragma unroll
+    for (int i = 0; i < XV; ++i)
+      xr[i] = *(const bf16x8*)(a.ma + (size_t)mid[MK ? i : 0] * a.r + c * GKC + ((threadIdx.x + i * GW * 64) & 15) * 8);
+  };
   auto load_x = [&](int c, bf16x8* xr) {
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
@@ -834,7 +886,8 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   };
   {
     bf16x8 xr[XV];
-    load_x(0, xr);
+    if constexpr (MK) load_xm(0, xr);
+    else load_x(0, xr);
     store_x(0, xr);
   }
   lds_barrier();
@@ -843,12 +896,15 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[mt][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int c, bf16x8 (&bq)[GPF][NT]) {
+  auto step = [&](int c, bf16x8 (&bq)[GPF][NT]) __attribute__((always_inline)) {
     // chunks past the end are clamped to the last: the x re-read lands in the idle LDS buffer,
     // which nothing reads again, and the weight re-read is never multiplied
     bf16x8 xr[XV];
-    load_x(min(c + 1, nchunks - 1), xr);
-    const int cw = min(c + 2, nchunks - 1);
+    if (MK && c + 1 < nm) load_xm(c + 1, xr);
+    else load_x(min(c + 1 - nm, nchunks - 1), xr);
+    const bf16x8* wn[NT];                             // chunk c + 2's fragments
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wn[t] = wchunk(c + 2, t);
     const uint16_t* xb = xs + (size_t)(c & 1) * ROWS * GKC + (size_t)(mh * MTW * 16 + (lane & 15)) * GKC;
 #pragma unroll
     for (int p = 0; p < GPF; ++p) {
@@ -873,40 +929,51 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
       // keep the reloads here: the scheduler would otherwise sink them to the end of the chunk
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) bq[p][t] = wload<PK>(wp[t] + (cw * GPF + p) * KS);
+      for (int t = 0; t < NT; ++t) bq[p][t] = frag(wn[t], p);
       __builtin_amdgcn_sched_barrier(0);
     }
     store_x((c + 1) & 1, xr);
     // LDS-only barrier: __syncthreads() would also wait for every weight fragment in flight
     lds_barrier();
   };
-  for (int c = 0; c < nchunks; c += 2) {
-    step(c, bqa);
-    if (c + 1 < nchunks) step(c + 1, bqb);
+  // the block's biases, as gemm_finish parks its logits (each element written and read by one lane)
+  constexpr int COLS = NG * NT * 16;
+  h16* const mb = (h16*)xs + gemm_lds<MT, NT, GW, MS>() / 2;
+  if constexpr (MK) {
+    for (int c = 0; c < nm; c += 2) {
+      step(c, bqa);
+      step(c + 1, bqb);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          mb[((mh * MTW + mt) * 16 + 4 * (lane >> 4) + q) * (COLS + 8) + ng * NT * 16 + t * 16 + (lane & 15)] =
+              (h16)acc[mt][t][q];
+        acc[mt][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
   }
-  gemm_finish<MTW, NT, NG * NT * 16, GW * 64, ROWS, F16>(a, acc, xs, mh * MTW, ng * NT * 16);
+  for (int c = nm; c < nm + nchunks; c += 2) {
+    step(c, bqa);
+    if (c + 1 < nm + nchunks) step(c + 1, bqb);
+  }
+  gemm_finish<MTW, NT, COLS, GW * 64, ROWS, F16, MK>(a, acc, mb, xs, mh * MTW, ng * NT * 16);
 }
 
-template <int MT, int NT, int GW, int MS>
-size_t gemm_lds() {
-  const size_t xbuf = 2 * (size_t)MT * 16 * GKC * 2;                      // x double buffer
-  const size_t lgt = (size_t)MT * 16 * (GW / MS * NT * 16 + 8) * 2 +      // the block's logits,
-                     ((size_t)MT * 16 + 1) * (KMAX * 4 + 8);              // staged winners' keys, (max, sum)
-  return xbuf > lgt ? xbuf : lgt;
-}
-
-template <int MT, int NT, int GW, bool PK, bool F16, int MS>
+template <int MT, int NT, int GW, bool PK, bool F16, int MS, bool MK = false>
 int launch_gemm(const GemmArgs& a0, hipStream_t st) {
   // cfh_head_ws_bytes sizes the candidate lists for blocks of at least 128 columns
   static_assert(GW / MS * NT * 16 >= 128, "a GEMM block must cover at least 128 shortlist columns");
   GemmArgs a = a0;
   const int cols = GW / MS * NT * 16;
   a.nsets = (a.n + cols - 1) / cols;
-  const size_t lds = gemm_lds<MT, NT, GW, MS>();
+  const size_t lds = gemm_lds<MT, NT, GW, MS>() + (MK ? (size_t)MT * 16 * (cols + 8) * 2 : 0);
   if (lds > 160 * 1024) return CFH_E_UNSUPPORTED;
-  CFH_HIP(hipFuncSetAttribute((const void*)k_head_gemm<MT, NT, GW, PK, F16, MS>,
+  CFH_HIP(hipFuncSetAttribute((const void*)k_head_gemm<MT, NT, GW, PK, F16, MS, MK>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL((k_head_gemm<MT, NT, GW, PK, F16, MS>), dim3(a.nsets), dim3(GW * 64), lds, st, a);
+  hipLaunchKernelGGL((k_head_gemm<MT, NT, GW, PK, F16, MS, MK>), dim3(a.nsets), dim3(GW * 64), lds, st, a);
   CFH_LAUNCH_CHECK();
   return CFH_OK;
 }
@@ -1585,6 +1652,29 @@ int cfh_head_gemm16_topk(const void* x, int M, int d, const void* packed, int n,
   if (cfh_head_packed_bytes(n, d, 0) < 0) return CFH_E_INVALID;
   return gemm_topk<true, true>(x, M, d, packed, nullptr, n, bias, k, logits, vals, ids, lse, ws,
                                (hipStream_t)stream);
+}
+
+int cfh_head_gemm16_markov_topk(const void* x, int M, int d, const void* packed, int n, const void* w1, int V,
+                                const int32_t* prev, int prev_stride, int r, int k, void* logits, float* vals,
+                                int32_t* ids, float* lse, void* ws, void* stream) {
+  const int64_t head_bytes = cfh_head_packed_bytes(n, d, 0);
+  if (head_bytes < 0 || cfh_head_packed_bytes(n, d, r) < 0 || r < 1) return CFH_E_INVALID;
+  if (!x || !packed || !w1 || !prev || prev_stride < 1 || V < 1 || M < 1 || d < GKC || d % GKC || n < 1 || k < 0 ||
+      k > KMAX || (k == 0 ? !logits : (!vals || !ids || !ws)))
+    return CFH_E_INVALID;
+  // (more rows' biases do not fit the LDS beside the operand buffers)
+  if (M > 128 || r % (2 * GKC)) return CFH_E_UNSUPPORTED;
+  GemmArgs ga = {};
+  ga.x = (const uint16_t*)x; ga.W = (const uint16_t*)packed; ga.logits = (uint16_t*)logits; ga.ws = ws;
+  ga.M = M; ga.d = d; ga.n = n; ga.k = k;
+  ga.mw = (const uint16_t*)((const char*)packed + head_bytes); ga.ma = (const uint16_t*)w1; ga.mids = prev;
+  ga.mid_stride = prev_stride; ga.r = r; ga.V = V;
+  hipStream_t st = (hipStream_t)stream;
+  const int nsets = gemm_nsets<8, 2, 8, 1>(n);       // (the same blocks at both row counts)
+  const int rc = M <= 64 ? launch_gemm<4, 2, 8, true, true, 1, true>(ga, st)
+                         : launch_gemm<8, 2, 8, true, true, 1, true>(ga, st);
+  if (rc || k == 0) return rc;
+  return launch_merge(ws, M, nsets, k, vals, ids, lse, st);
 }
 
 int64_t cfh_path_ws_bytes(int M, int d, int ffn_mult, int order) {

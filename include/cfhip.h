@@ -119,8 +119,8 @@ int cfh_flow_pack_expert(const cfh_flow_dims* dims, const void* const* raw, int 
  *   z_out   : [batch][draft_length][d] fp16 predicted hiddens
  *   ws      : workspace of cfh_caps(dims, batch) bytes
  * A batch runs in groups of requests whose rows share every weight stream: up to sixteen (wide
- * groups, rows staged in K chunks; head width a multiple of 128 and the folded cross attention),
- * else up to two (both drafts in one 16-row MFMA tile); cfh_flow_group_size tells.
+ * groups, rows staged in K chunks), or two (both drafts in one 16-row MFMA tile, or a wide group
+ * where their rows do not fit it); cfh_flow_group_size tells.
  * Chunk experts (d >= 1024, two or more chunks) run their Euler steps on companion streams of the
  * caller's stream, forked after the per-draft launches and joined before return.  The first eager
  * call on a caller stream without companions creates them (streams, events: kept until
@@ -348,6 +348,15 @@ int cfh_head_topk_grouped(const void* h, int G, int M, int d, const void* W, con
  * log_softmax / topk over B*n rows (cf/vllm_plugin/flow_proposer.py:1021-1025, 1142-1165). */
 int cfh_head_gemm16_topk(const void* x, int M, int d, const void* packed, int n, const void* bias, int k,
                          void* logits, float* vals, int32_t* ids, float* lse, void* ws, void* stream);
+
+/* cfh_head_gemm16_topk with the markov bias computed in the same launch, bit for bit as with the k = 0
+ * logits of the markov rows passed as its bias: logits[m][j] = fp16( fp16(x[m] . W[row_j]) +
+ * fp16(w1[prev_m] . w2[row_j]) ), prev_m = prev[m * prev_stride] clamped to [0, V).  packed: a
+ * cfh_head_pack image of n rows with its markov rows; w1 [V][r] fp16; r % 256 == 0, M <= 128
+ * (CFH_E_UNSUPPORTED past them: take the two calls). */
+int cfh_head_gemm16_markov_topk(const void* x, int M, int d, const void* packed, int n, const void* w1, int V,
+                                const int32_t* prev, int prev_stride, int r, int k, void* logits, float* vals,
+                                int32_t* ids, float* lse, void* ws, void* stream);
 
 /* ---------------------------------------------------------------- draft search
  * Path-conditioned residual of the PathHead, fused form (cf/vllm_plugin/fused.py:25-37;

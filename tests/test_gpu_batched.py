@@ -40,6 +40,40 @@ def _bound(h64, w64, ref):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,n,d,stride", [(9, 777, 256, 1), (64, 1024, 512, 4), (65, 1000, 256, 1), (128, 300, 768, 3)])
+def test_gemm16_markov_equals_two_calls(cuda, M, n, d, stride):
+    """The markov bias computed inside the head's launch (up to 128 rows) against the bias as a launch of
+    its own: logits, top-k and log-sum-exp bit for bit, at both row counts' edges, ragged shortlists,
+    odd and even counts of head chunks and strided parents (one of them absent: -1 reads row 0)."""
+    from chain_flow_amd import _lib
+    g = torch.Generator().manual_seed(M + n)
+    V, r = 1500, 256
+    lm, w1, w2 = (torch.randn(V, x, generator=g).mul(0.1).half().to(cuda) for x in (d, r, r))
+    sl = torch.randperm(V, generator=g)[:n].sort().values.to(torch.int32).to(cuda)
+    head = ShortlistHead(lm, sl, w1, w2)
+    h = torch.randn(M, d, generator=g).half().to(cuda)
+    prev = torch.randint(0, V, (M, stride), generator=g, dtype=torch.int32).to(cuda)
+    prev[M // 2, 0] = -1
+    got_l, ref_l = (torch.empty(M, n, dtype=torch.float16, device=cuda) for _ in range(2))
+    print(f"[gemm16 markov] M={M} n={n} d={d} stride={stride}", flush=True)
+    got = head.topk(h, 4, prev=prev.view(-1), prev_stride=stride, logits=got_l)
+    L, st = _lib.lib(), _lib.stream_handle()
+    a = w1.index_select(0, prev[:, 0].clamp_min(0).long())
+    bias = torch.empty(M, n, dtype=torch.float16, device=cuda)
+    w2img = head.image.data_ptr() + int(L.cfh_head_packed_bytes(n, d, 0))
+    _lib.check(L.cfh_head_gemm16_topk(a.data_ptr(), M, r, w2img, n, None, 0, bias.data_ptr(), None, None, None, None,
+                                      st), "markov")
+    vals, ids, lse = (torch.empty(M, 4, device=cuda), torch.empty(M, 4, dtype=torch.int32, device=cuda),
+                      torch.empty(M, device=cuda))
+    _lib.check(L.cfh_head_gemm16_topk(h.data_ptr(), M, d, head.image.data_ptr(), n, bias.data_ptr(), 4,
+                                      ref_l.data_ptr(), vals.data_ptr(), ids.data_ptr(), lse.data_ptr(),
+                                      head.workspace(M, 4, cuda).data_ptr(), st), "head")
+    torch.cuda.synchronize()
+    assert torch.equal(got_l, ref_l) and torch.equal(got[0], vals) and torch.equal(got[1], ids)
+    assert torch.equal(got[2], lse)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,n,markov", [(9, 1024, True), (40, 1000, False), (160, 1024, True), (256, 777, True)])
 def test_gemm16_head_matches_oracle(cuda, M, n, markov):
     cfg, W, _ = _setup(n=n)
