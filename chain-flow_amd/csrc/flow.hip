@@ -291,12 +291,18 @@ struct XattArgs {
   int nex, d, H, C, nb;  // C: context rows of all the group's requests (the most of any entry)
   int Cq;                // context rows per request: row r scores only its request's rows
   int nsg, Csg;          // subgroups, context rows per subgroup (0: C)
+  int cv;                // columns a thread: 4 (the wide groups) or 1
   float scale;
 };
 
 constexpr int XT = 512;        // threads of an XATT workgroup
 
-template <int CM>              // context rows, padded to 8 or 16
+// CM: context rows, padded to 8 or 16.  CV: adjacent columns a thread.  At 4 (the wide groups, whose
+// subgroups fill the chip) a thread reads each row of P_h once for its four columns, only the half
+// that holds its request's context rows, and the scores are computed for up to 2,048 columns at
+// once: with columns XT apart, one at a time over all 16 context rows, the LDS reads of P_h bound the
+// launch.  Two 16-request groups at d = 4096: 33.6 -> 31.4 us; 13 requests at d = 2560: 16.1 -> 11.6 us.
+template <int CM, int CV>
 __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
   constexpr int NW = XT / 64;
   constexpr int XRS = CM == 8 ? 20 : 10;     // k-steps a wave loads in one round (registers)
@@ -317,11 +323,12 @@ __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // this thread's first column of B_h (every context row of the subgroup), in flight before the
   // scores; a block of more than XT columns gives the thread further columns XT apart
-  const int cpb = d / a.nb, n = cb * cpb + min(t, cpb - 1);
+  typedef h16 hv __attribute__((ext_vector_type(CV)));
+  const int cpb = d / a.nb, n = cb * cpb + min(t * CV, cpb - CV);
   const h16* Bbase = a.Bf[e] + ((size_t)h * Ct + c0) * d;
-  h16 bv[CM];
+  hv bv[CM];
 #pragma unroll
-  for (int c = 0; c < CM; ++c) bv[c] = Bbase[(size_t)min(c, C - 1) * d + n];
+  for (int c = 0; c < CM; ++c) bv[c] = *(const hv*)(Bbase + (size_t)min(c, C - 1) * d + n);
   // scores: lane row = lane % 16, context row = lane % 16 of the B operand, k-group lane / 16.
   // Lanes of rows past S or context rows past C load nothing (zero operands).  The operand
   // images hold every row of the expert (St) and every context row (Ct).
@@ -370,22 +377,48 @@ __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
   }
   __syncthreads();
   // this thread's columns of P_h B_h
-  for (int cc = t; cc < cpb; cc += XT) {
-    const int nn = cb * cpb + cc;
-    float* oh = a.out[e] + ((size_t)h * St + r0) * d + nn;
-    float bf[CM];
-    if (cc == t) {
+  if constexpr (CV == 4) {
+    if (t * CV >= cpb) return;
+    float* oh = a.out[e] + ((size_t)h * St + r0) * d + n;
+    // rows [ra, rb) over context rows [LO, LO + NC)
+    auto rows = [&](int ra, int rb, auto lo, auto nc) __attribute__((always_inline)) {
+      constexpr int LO = decltype(lo)::value, NC = decltype(nc)::value;
+      f32x4 bf[NC];
 #pragma unroll
-      for (int c = 0; c < CM; ++c) bf[c] = (float)bv[c];
+      for (int c = 0; c < NC; ++c)
+        bf[c] = (f32x4){(float)bv[LO + c][0], (float)bv[LO + c][1], (float)bv[LO + c][2], (float)bv[LO + c][3]};
+      for (int r = ra; r < rb; ++r) {
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) o += P[r][LO + c] * bf[c];
+        *(f32x4*)(oh + (size_t)r * d) = o;
+      }
+    };
+    if (CM == 16 && a.Cq == 8) {                     // a request's rows over its own context rows
+      rows(0, min(S, a.Sr[e]), std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{});
+      rows(a.Sr[e], S, std::integral_constant<int, CM == 16 ? 8 : 0>{}, std::integral_constant<int, 8>{});
     } else {
-#pragma unroll
-      for (int c = 0; c < CM; ++c) bf[c] = (float)Bbase[(size_t)min(c, C - 1) * d + nn];
+      rows(0, S, std::integral_constant<int, 0>{}, std::integral_constant<int, CM>{});
     }
-    for (int r = 0; r < S; ++r) {
-      float o = 0.f;
+    return;
+  } else {
+    for (int cc = t; cc < cpb; cc += XT) {
+      const int nn = cb * cpb + cc;
+      float* oh = a.out[e] + ((size_t)h * St + r0) * d + nn;
+      float bf[CM];
+      if (cc == t) {
 #pragma unroll
-      for (int c = 0; c < CM; ++c) o += P[r][c] * bf[c];
-      oh[(size_t)r * d] = o;
+        for (int c = 0; c < CM; ++c) bf[c] = (float)bv[c][0];
+      } else {
+#pragma unroll
+        for (int c = 0; c < CM; ++c) bf[c] = (float)Bbase[(size_t)min(c, C - 1) * d + nn];
+      }
+      for (int r = 0; r < S; ++r) {
+        float o = 0.f;
+#pragma unroll
+        for (int c = 0; c < CM; ++c) o += P[r][c] * bf[c];
+        oh[(size_t)r * d] = o;
+      }
     }
   }
 }
@@ -456,12 +489,11 @@ __global__ void __launch_bounds__(1024) k_xbias(XbiasArgs a) {
 // Column blocks per (expert, head) of XATT: the fewest that give each thread at most one column
 // (each block recomputes the head's scores, so more blocks only repeat that work); 0 if d has no
 // such split.
-// cols: the most columns a thread may take (each block recomputes its head's scores: the wide
-// groups' many subgroups already fill the chip, so there a thread takes several columns).
-int xattn_blocks(int d, int units, int cols = 1) {
-  (void)units;
+// cv: columns a thread takes (each block recomputes its head's scores: the wide groups' many
+// subgroups already fill the chip, so there a thread takes four adjacent columns).
+int xattn_blocks(int d, int cv = 1) {
   for (int nb = 1; nb <= d; ++nb)
-    if (d % nb == 0 && d / nb <= XT * cols && (d / nb <= XT || (d / nb) % XT == 0)) return nb;
+    if (d % nb == 0 && d / nb % cv == 0 && d / nb <= XT * cv) return nb;
   return 0;
 }
 
@@ -473,8 +505,14 @@ int launch_xattn(const XattArgs& a, hipStream_t st) {
     if (Ssg > MAXR || (long long)a.nsg * Ssg < a.S[e]) return CFH_E_UNSUPPORTED;
   }
   const dim3 grid((unsigned)(a.nex * a.H * a.nsg * a.nb));
-  if (Csg <= 8) hipLaunchKernelGGL(k_xattn<8>, grid, dim3(XT), 0, st, a);
-  else hipLaunchKernelGGL(k_xattn<16>, grid, dim3(XT), 0, st, a);
+  if (a.cv == 4) {
+    if (a.d / a.nb % 4 || a.d / a.nb > 4 * XT) return CFH_E_UNSUPPORTED;
+    if (Csg <= 8) hipLaunchKernelGGL((k_xattn<8, 4>), grid, dim3(XT), 0, st, a);
+    else hipLaunchKernelGGL((k_xattn<16, 4>), grid, dim3(XT), 0, st, a);
+  } else {
+    if (Csg <= 8) hipLaunchKernelGGL((k_xattn<8, 1>), grid, dim3(XT), 0, st, a);
+    else hipLaunchKernelGGL((k_xattn<16, 1>), grid, dim3(XT), 0, st, a);
+  }
   CFH_LAUNCH_CHECK();
   return CFH_OK;
 }
@@ -869,7 +907,7 @@ void make_wide_plan(Plan& p, const cfh_flow_dims* dm) {
   p.pks = p.fold ? p.H : 1;
   for (const WideShape& w : p.ws)
     if (w.ok) p.pks = std::max({p.pks, w.ks_wo, w.ks_ww2, w.ks_wout, w.ks_oc});
-  p.xnb = p.fold ? xattn_blocks(p.d, p.nch * p.H, 4) : 0;
+  p.xnb = p.fold ? xattn_blocks(p.d, 4) : 0;
   p.ok = p.ws[0].ok && (!p.fold || p.xnb > 0) &&
          (size_t)3 * p.KD * p.hd * 2 + (size_t)p.KD * p.KD * 4 <= 64 * 1024 &&   // self attention's LDS
          (p.fold || cross_attn_lds(p.KD, p.C, p.hd) <= 64 * 1024);
@@ -936,7 +974,7 @@ Plan make_plan(const cfh_flow_dims* dm, int R = 1, bool wide = false) {
   if (p.fold) p.pks = std::max(p.pks, p.H);   // the folded cross attention's per-head partials
   if (p.fold) {
     p.wpb_fold = wpb_for_grid(tiles_d, 2 * p.nch * p.ks_fold, 8, p.S_fold * (p.d / p.ks_fold) / 8);
-    p.xnb = xattn_blocks(p.d, p.nch * p.H);
+    p.xnb = xattn_blocks(p.d);
   }
   p.ok = p.ks_qc > 0 && p.ks_qc <= 8 && p.ks_w2 > 0 && p.ks_out > 0 && p.ks_att > 0 && res_nq(p.d) > 0 &&
          p.Smax <= MAXR && p.Ct <= 16;
@@ -1349,6 +1387,7 @@ int block_pass_wide(const Plan& p, const WideShape& sh, const cfh::ExpertLayout&
     XattArgs x = {};
     x.nex = nex; x.d = d; x.H = p.H; x.Cq = p.C; x.nb = p.xnb; x.scale = 1.0f / sqrtf((float)p.hd);
     x.Csg = 2 * p.C;
+    x.cv = 4;
     for (int g = 0; g < ng; ++g) {
       const int Cg = gr[g].Rg * p.C;
       const size_t per_l = (size_t)p.H * Cg * d;
