@@ -913,8 +913,7 @@ void make_wide_plan(Plan& p, const cfh_flow_dims* dm) {
          (p.fold || cross_attn_lds(p.KD, p.C, p.hd) <= 64 * 1024);
 }
 
-// wide: the wide plan also where R requests' rows fit one 16-row tile.
-Plan make_plan(const cfh_flow_dims* dm, int R = 1, bool wide = false) {
+Plan make_plan(const cfh_flow_dims* dm, int R = 1) {
   Plan p = {};
   p.d = dm->d; p.fd = dm->ffn_mult * dm->d; p.CS = dm->chunk_size; p.E = dm->flow_steps;
   p.NL = dm->layers; p.C = dm->ctx_rows; p.KD = dm->draft_length; p.H = dm->heads; p.hd = p.d / p.H;
@@ -925,7 +924,7 @@ Plan make_plan(const cfh_flow_dims* dm, int R = 1, bool wide = false) {
   p.Smax = R * p.KD;
   const int out_rows = R == 1 ? p.CS : p.Smax;   // OUT: the current chunk's rows, or every row when packed
   p.res_mode = dm->numerics == CFH_FLOW_MODULES ? RES_ADD16 : RES_ADD32;
-  if (p.Smax > MAXR || wide) {
+  if (p.Smax > MAXR) {
     make_wide_plan(p, dm);
     return p;
   }
@@ -1012,30 +1011,19 @@ Plan make_plan(const cfh_flow_dims* dm, int R = 1, bool wide = false) {
   return p;
 }
 
-// Plan of a batch, its requests per group in it.  Wide groups (allow_wide, more than two requests): the
-// batch in as few groups of at most WMAXR / draft_length requests as possible, balanced; otherwise
-// the most requests (up to `batch`) whose rows fit one 16-row tile and whose plan this build runs, or,
-// where no such plan fits (d = 5120: 16 rows of it exceed the LDS), one wide group of them all: two
-// requests at d = 5120, L = 8, E = 8 took 38.4 ms one after the other, 20.0 ms as a wide group.
-// One request a group always works when the shape is supported.
-Plan batch_plan(const cfh_flow_dims* dm, int batch, bool allow_wide = true) {
+// Requests per group for a batch.  Wide groups (allow_wide, more than two requests): the batch in
+// as few groups of at most WMAXR / draft_length requests as possible, balanced; otherwise the
+// most requests (up to `batch`) whose rows fit one 16-row tile and whose plan this build runs.
+// 1 always works when the shape is supported.
+int group_size(const cfh_flow_dims* dm, int batch, bool allow_wide = true) {
   const int KD = dm->draft_length;
   if (allow_wide && batch * KD > MAXR && WMAXR / KD >= 3) {
     const int rmax = WMAXR / KD, ng = (batch + rmax - 1) / rmax, R = (batch + ng - 1) / ng;
-    if (R * KD > MAXR) {
-      const Plan p = make_plan(dm, R);
-      if (p.ok) return p;
-    }
+    if (R * KD > MAXR && make_plan(dm, R).ok) return R;
   }
-  for (int R = std::min(batch, MAXR / KD); R > 1; --R) {
-    const Plan p = make_plan(dm, R);
-    if (p.ok) return p;
-  }
-  if (allow_wide && batch > 1 && batch * KD <= MAXR) {
-    const Plan p = make_plan(dm, batch, true);
-    if (p.ok) return p;
-  }
-  return make_plan(dm, 1);
+  for (int R = std::min(batch, MAXR / KD); R > 1; --R)
+    if (make_plan(dm, R).ok) return R;
+  return 1;
 }
 
 struct WS {
@@ -1660,7 +1648,7 @@ size_t group_ws_stride(const Plan& p) { return cfh::align256(carve(p, nullptr).t
 
 // Workspace of a batch: one group's, or two groups' when the wide path pairs them.
 size_t flow_ws_bytes(const cfh_flow_dims* dm, int batch) {
-  const Plan p = batch_plan(dm, batch);
+  const Plan p = make_plan(dm, group_size(dm, batch));
   if (!p.ok) return 0;
   if (p.wide && (batch + p.R - 1) / p.R > 1 && p.ws[1].ok) return 2 * group_ws_stride(p);
   return carve(p, nullptr).total;
@@ -2090,7 +2078,7 @@ extern "C" {
 int cfh_caps(const cfh_flow_dims* dims, int batch, int64_t* ws_bytes) {
   if (!cfh::flow_dims_ok(dims) || batch < 1) return CFH_E_UNSUPPORTED;
   if (dims->d > ROWT * ROWE || dims->draft_length > MAXR) return CFH_E_UNSUPPORTED;
-  const Plan p = batch_plan(dims, batch);
+  const Plan p = make_plan(dims, group_size(dims, batch));
   if (!p.ok) return CFH_E_UNSUPPORTED;
   // the workspace of every batch up to `batch`: the group sizes 1, 2 (narrow), the widest single
   // group, two of them (wide group sizes grow with the batch up to WMAXR / draft_length requests;
@@ -2110,9 +2098,9 @@ int cfh_flow_group_size(const cfh_flow_dims* dims, int batch, int* requests) {
   *requests = 0;
   if (!cfh::flow_dims_ok(dims) || batch < 1) return CFH_E_UNSUPPORTED;
   if (dims->d > ROWT * ROWE || dims->draft_length > MAXR) return CFH_E_UNSUPPORTED;
-  const Plan p = batch_plan(dims, batch);
-  if (!p.ok) return CFH_E_UNSUPPORTED;
-  *requests = p.R;
+  const int R = group_size(dims, batch);
+  if (!make_plan(dims, R).ok) return CFH_E_UNSUPPORTED;
+  *requests = R;
   return CFH_OK;
 }
 
@@ -2121,7 +2109,7 @@ int cfh_flow_plan(const cfh_flow_dims* dims, int batch, int* flags) {
   *flags = 0;
   if (!cfh::flow_dims_ok(dims) || batch < 1) return CFH_E_UNSUPPORTED;
   if (dims->d > ROWT * ROWE || dims->draft_length > MAXR) return CFH_E_UNSUPPORTED;
-  const Plan p = batch_plan(dims, batch);
+  const Plan p = make_plan(dims, group_size(dims, batch));
   if (!p.ok) return CFH_E_UNSUPPORTED;
   *flags = (p.fold ? CFH_PLAN_FOLD : 0) | (p.fold2 ? CFH_PLAN_FOLD2 : 0) | (p.xblk ? CFH_PLAN_XBLK : 0) |
            (p.wide ? CFH_PLAN_WIDE : 0) | (p.conc ? CFH_PLAN_CONC : 0);
@@ -2132,7 +2120,7 @@ int cfh_flow_integrate(const cfh_flow_dims* dm, const void* const* experts, cons
                        void* ws_ptr, int batch, void* stream) {
   if (!cfh::flow_dims_ok(dm) || dm->d > ROWT * ROWE || dm->draft_length > MAXR) return CFH_E_UNSUPPORTED;
   if (!experts || !ctx || !z_out || !ws_ptr || batch < 1) return CFH_E_INVALID;
-  const Plan p = batch_plan(dm, batch);
+  const Plan p = make_plan(dm, group_size(dm, batch));
   if (!p.ok) return CFH_E_UNSUPPORTED;
   for (int c = 0; c < p.nch; ++c)
     if (!experts[c]) return CFH_E_INVALID;
@@ -2143,7 +2131,7 @@ int cfh_flow_integrate_anchored(const cfh_flow_dims* dm, const void* const* expe
                                 const void* anchor, void* z_out, void* ws_ptr, int batch, void* stream) {
   if (!cfh::flow_dims_ok(dm) || dm->d > ROWT * ROWE || dm->draft_length > MAXR) return CFH_E_UNSUPPORTED;
   if (!experts || !ctx || !anchor || !z_out || !ws_ptr || batch < 1) return CFH_E_INVALID;
-  const Plan p = batch_plan(dm, batch);
+  const Plan p = make_plan(dm, group_size(dm, batch));
   if (!p.ok) return CFH_E_UNSUPPORTED;
   for (int c = 0; c < p.nch; ++c)
     if (!experts[c]) return CFH_E_INVALID;
@@ -2199,7 +2187,7 @@ int cfh_flow_integrate_noalloc(const cfh_flow_dims* dm, const void* const* exper
   if (!cfh::flow_dims_ok(dm) || dm->d > ROWT * ROWE || dm->draft_length > MAXR) return CFH_E_UNSUPPORTED;
   if (!experts || !ctx || !z_out || batch < 1) return CFH_E_INVALID;
   // narrow groups (at most two requests a weight stream): their workspace fits the scratch array
-  const Plan p = batch_plan(dm, batch, false);
+  const Plan p = make_plan(dm, group_size(dm, batch, false));
   if (!p.ok) return CFH_E_UNSUPPORTED;
   for (int c = 0; c < p.nch; ++c)
     if (!experts[c]) return CFH_E_INVALID;

@@ -236,13 +236,12 @@ def test_packed_batch_matches_oracle_per_request(cuda, d, B, layers):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("d,B", [(256, 8), (256, 9), (256, 16), (4096, 31), (5120, 2)])
+@pytest.mark.parametrize("d,B", [(256, 8), (256, 9), (256, 16), (4096, 31)])
 def test_wide_groups_at_row_group_edges_match_oracle(cuda, d, B):
     """Wide launches at the edges of their row groups and workgroup shapes: 32 and 64 rows an expert
     (whole row groups, the first expert multiplying half of them), 36 and 72 (a part of the third,
     the fifth), 64 and 128 (the most); 4096 x 31 pairs groups of 16 and 15 requests in the 8-wave and
-    three-tile shapes; 5120 x 2 is one wide group because two requests' rows of that width do not fit
-    the narrow kernel's LDS.  Each request against the oracle on its own context."""
+    three-tile shapes.  Each request against the oracle on its own context."""
     cfg = flownet(d, layers=1, flow_steps=1 if d > 1024 else 2)
     assert plan_flags(cfg, B) & _lib.PLAN_WIDE
     W = _flow_weights(cfg, seed=19)
@@ -250,7 +249,7 @@ def test_wide_groups_at_row_group_edges_match_oracle(cuda, d, B):
     print(f"[flow wide edges] d={d} B={B}", flush=True)
     ff = FusedFlow(cfg, {k: v.to(cuda) for k, v in W.items()}, device=cuda)
     z = to64(ff.predict_hidden(ctx.to(cuda)))
-    check = range(B) if d != 4096 else (0, 15, 16, 30)
+    check = range(B) if d <= 1024 else (0, 15, 16, 30)
     ref = oflow.predict_hidden(weights64(W), to64(ctx)[list(check)], _ocfg(cfg), numerics="fp16_modules")
     e = [rel_err(z[b:b + 1], ref[i:i + 1]) for i, b in enumerate(check)]
     print(f"  worst request {max(e):.3e}", flush=True)
