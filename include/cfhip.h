@@ -119,8 +119,8 @@ int cfh_flow_pack_expert(const cfh_flow_dims* dims, const void* const* raw, int 
  *   z_out   : [batch][draft_length][d] fp16 predicted hiddens
  *   ws      : workspace of cfh_caps(dims, batch) bytes
  * A batch runs in groups of requests whose rows share every weight stream: up to sixteen (wide
- * groups, rows staged in K chunks), or two (both drafts in one 16-row MFMA tile, or a wide group
- * where their rows do not fit it); cfh_flow_group_size tells.
+ * groups, rows staged in K chunks), else up to two (both drafts in one 16-row MFMA tile);
+ * cfh_flow_group_size tells.
  * Chunk experts (d >= 1024, two or more chunks) run their Euler steps on companion streams of the
  * caller's stream, forked after the per-draft launches and joined before return.  The first eager
  * call on a caller stream without companions creates them (streams, events: kept until
