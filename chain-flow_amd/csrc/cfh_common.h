@@ -50,6 +50,16 @@ __device__ __forceinline__ float gelu_erf(float x) {
   return x * (x < 0.f ? q : 1.0f - q);
 }
 
+// The path head's erf-GELU, fp16(0.5 x (1 + erff(x / sqrt 2))), the product rounded once: its rows go
+// straight into a 16-bit top-k, whose near ties other last bits would order differently.  (Written out as
+// the instruction because the compiler rounds the product to float first where it stores two results at
+// once: 0.1% of the hiddens' elements then move by one fp16 step.)
+__device__ __forceinline__ h16 gelu16_erff(float x) {
+  h16 y;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(y) : "v"(0.5f * x), "v"(1.0f + erff(x * 0.70710678118654752440f)));
+  return y;
+}
+
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 
 // Cross-lane steps by DPP (a VALU operand modifier, a few cycles) rather than __shfl_xor, which

@@ -20,7 +20,7 @@ constexpr int PF_SPLIT = 8;       //                                   split-K k
 constexpr int STREAM_SYNC = 4;    // fragment groups between workgroup barriers in the stream (measured: 4 best of 0-4)
 
 enum SrcKind { S_BUF = 0, S_SELF = 1, S_CROSS = 2 };
-enum EpiKind { E_PART = 0, E_BIAS16 = 1, E_GELU16 = 2, E_PART16 = 3 };
+enum EpiKind { E_PART = 0, E_BIAS16 = 1, E_GELU16 = 2, E_PART16 = 3, E_GELUF16 = 4 };
 
 struct SEx {
   const h16x8* w;      // packed weights: fragment (tile t, k-step s) at ((t * K/32) + s) * 64

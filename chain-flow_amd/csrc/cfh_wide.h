@@ -39,7 +39,7 @@ struct WEx {
   const h16x8* w;      // packed weights: fragment (tile t, k-step s) at ((t * K/32) + s) * 64
   const h16* a;        // activation rows [S][lda]; the unit's K range [kc K/ks, (kc+1) K/ks) is read
   int lda;
-  const h16* bias;     // E_BIAS16 / E_GELU16 bias [N]
+  const h16* bias;     // E_BIAS16 / E_GELU16 / E_GELUF16 bias [N]
   void* out;           // E_PART: float [ks][S][N]; E_PART16: h16 (as SEx); otherwise h16 (below)
   int S;               // activation rows (1 .. WMAXR)
   int pack, hrows;     // E_PART16: as SEx
@@ -51,7 +51,7 @@ struct WEx {
 struct WArgs {
   WEx ex[4];
   int nex, N, K, ks, wg_per_kc;
-  int gelu_r16;        // E_GELU16: as SArgs
+  int gelu_r16;        // E_GELU16: as SArgs (E_GELUF16: gelu16_erff of the rounded sum)
   int pair;            // entries e and e + nex/2 stream the same weights (two request groups of one
                        // expert): their workgroups for a unit run side by side on one XCD
   int map;             // workgroup order (set by launch_wide): MAP_PLAIN, MAP_PAIR or MAP_XCD
@@ -156,7 +156,7 @@ __device__ __forceinline__ void wide_unit(const WArgs& a, const WEx& ex, int kc,
   // cbase + q of the tile, so that a lane stores four adjacent columns at once
   const int row = lane & 15, kg = lane >> 4, cbase = 4 * kg;
   h16x4 bias[WT];
-  if constexpr (EPI == E_BIAS16 || EPI == E_GELU16) {
+  if constexpr (EPI == E_BIAS16 || EPI == E_GELU16 || EPI == E_GELUF16) {
 #pragma unroll
     for (int u = 0; u < WT; ++u)
 #pragma unroll
@@ -253,7 +253,8 @@ __device__ __forceinline__ void wide_unit(const WArgs& a, const WEx& ex, int kc,
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const float y = v[q] + (float)bias[u][q];
-          w[q] = EPI == E_BIAS16 ? (h16)y : (h16)gelu_erf(a.gelu_r16 ? r16(y) : y);
+          if constexpr (EPI == E_GELUF16) w[q] = gelu16_erff(r16(y));
+          else w[q] = EPI == E_BIAS16 ? (h16)y : (h16)gelu_erf(a.gelu_r16 ? r16(y) : y);
         }
         h16* o = (h16*)ex.out + (size_t)r * a.N + n;
         if (EPI == E_BIAS16 && ex.nsplit > 0) {
@@ -401,9 +402,10 @@ int launch_wide(const WArgs& a0, WShape s, hipStream_t st) {
   }
 #define CFH_WIDE(W, T, R) CFH_WIDE_S(2, W, T, R) CFH_WIDE_S(4, W, T, R) CFH_WIDE_S(8, W, T, R)
   CFH_WIDE(4, 2, 1)
-  // (the factor launches and the gathered ones come in one shape only)
+  // (the factor launches come in one shape only, the gathered ones in two)
+  if constexpr (EPI != E_PART16) { CFH_WIDE(8, 2, 1) }
   if constexpr (EPI != E_PART16 && !GA) {
-    CFH_WIDE(4, 1, 2) CFH_WIDE(4, 1, 1) CFH_WIDE(4, 3, 1) CFH_WIDE(8, 2, 1) CFH_WIDE(8, 3, 1)
+    CFH_WIDE(4, 1, 2) CFH_WIDE(4, 1, 1) CFH_WIDE(4, 3, 1) CFH_WIDE(8, 3, 1)
   }
 #undef CFH_WIDE
 #undef CFH_WIDE_S

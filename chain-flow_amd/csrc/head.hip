@@ -1127,7 +1127,7 @@ __global__ void __launch_bounds__(WK * 64) k_path_gemv(PathGemvArgs g) {
     const int m = rbase + j;
     if (m >= g.M) continue;
     if constexpr (EPI == PG_GELU) {
-      g.out[(size_t)m * g.N + n] = (h16)gelu_erf(r16(v[j] + b));
+      g.out[(size_t)m * g.N + n] = gelu16_erff(r16(v[j] + b));
     } else {
       const int grp = g.rows_per_pred > 0 ? (g.row0 + m) / g.rows_per_pred : 0;
       g.out[(size_t)m * g.N + n] = (h16)((float)g.pred[(size_t)grp * g.pred_ld + n] + r16(v[j] + b));
@@ -1198,14 +1198,22 @@ PathPlan path_plan(int M, int d, int ffn, int order) {
   return p;
 }
 
+// Workgroup shape of a split-K launch of `units` units: eight 16-column tiles in four waves, or, where
+// those would come to more than one workgroup a CU and the operand buffers of more than 64 rows leave
+// room for only one at a time, sixteen in eight.  128 rows, four offsets: d = 5120, 320 workgroups of four
+// waves 75.6 us, 160 of eight 62.1 (down-projection 47.1 and 39.9); d = 2560 27.7 and 24.0 (21.5 and
+// 18.6).  (The tiles only share out the columns: the sums are the same in both.)
+WShape path_split(int M, int N, int units, int ks) {
+  const long long wgs = (long long)units * (N / 16 / 8) * ks;
+  return M > 64 && wgs > 256 && N / 16 % 16 == 0 ? WShape{8, 2, 1} : WShape{4, 2, 1};
+}
+
 // The path residual of many rows (the beams of a batch) in groups of up to WMAXR rows: every weight
 // of the path head streams once per group through the wide kernel (cfh_wide.h) instead of once
 // per 16 rows.  offsets: one k_wide launch over the live offset projections (the embedding rows
 // gathered by the ancestor ids), split-K partials; k_path_sum; up: k_wide with the GELU epilogue
 // (fp16 rounding before the GELU, as torch's Linear then GELU modules); down: split-K partials;
 // k_path_out.
-constexpr WShape PATH_SPLIT = {4, 2, 1};   // workgroup shape of the split-K launches
-
 struct PathWide {
   bool ok;
   int o_ks, dn_ks;
@@ -1216,16 +1224,29 @@ struct PathWide {
 PathWide path_wide_plan(int M, int d, int ffn, int order) {
   PathWide p = {};
   const int pf = ffn * d;
-  p.o_ks = wide_ks(d, d, order, PATH_SPLIT);
-  p.dn_ks = wide_ks(d, pf, 1, PATH_SPLIT);
+  // k-splits: the first to give 256 workgroups of eight tiles.  The flow's rule (wide_ks: the most
+  // workgroups up to 256) adds the partials of d = 2560 and 5120 in another order: 12% of the hiddens'
+  // elements then move by one fp16 step, and up to 1.2% of a depth's ids swap where 16-bit logits nearly tie
+  constexpr int CUS = 256;
+  auto ks_for = [&](int units, int N, int K) {
+    int best = 0;
+    for (int ks = 1; ks <= K / WCH; ++ks) {
+      if (K % ks || (K / ks) % WCH) continue;
+      best = ks;
+      if ((long long)units * (N / 16 / 8) * ks >= CUS) break;
+    }
+    return best;
+  };
+  p.o_ks = ks_for(order, d, d);
+  p.dn_ks = ks_for(1, d, pf);
   p.up = wide_shape_for(pf / 16, 1);
   auto wa = [&](int nex, int N, int K, int ks) {
     WArgs a = {};
     a.nex = nex; a.N = N; a.K = K; a.ks = ks;
     return a;
   };
-  p.ok = order <= 4 && p.o_ks > 0 && p.dn_ks > 0 && p.up.wv > 0 && !wide_check(wa(order, d, d, p.o_ks), PATH_SPLIT, M) &&
-         !wide_check(wa(1, pf, d, 1), p.up, M) && !wide_check(wa(1, d, pf, p.dn_ks), PATH_SPLIT, M);
+  p.ok = order <= 4 && p.o_ks > 0 && p.dn_ks > 0 && p.up.wv > 0 && !wide_check(wa(order, d, d, p.o_ks), WShape{4, 2, 1}, M) &&
+         !wide_check(wa(1, pf, d, 1), p.up, M) && !wide_check(wa(1, d, pf, p.dn_ks), WShape{4, 2, 1}, M);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -1707,7 +1728,7 @@ static int path_group_wide(const PathWide& pw, const void* const* ph, int order,
       x.w = (const h16x8*)ph[j]; x.a = (const h16*)embed_w; x.lda = d; x.ids = lastp + j; x.ids_stride = order;
       x.out = P + (size_t)j * pw.o_ks * M * d; x.S = M;
     }
-    if ((rc = launch_wide<E_PART, false, WCH, true>(a, PATH_SPLIT, st))) return rc;
+    if ((rc = launch_wide<E_PART, false, WCH, true>(a, path_split(M, d, o, pw.o_ks), st))) return rc;
   }
   PathSumArgs ps = {};
   ps.P = P; ps.lastp = lastp; ps.g = (const h16*)ph[2 * order]; ps.b = (const h16*)ph[2 * order + 1]; ps.a = A;
@@ -1717,16 +1738,16 @@ static int path_group_wide(const PathWide& pw, const void* const* ph, int order,
   CFH_LAUNCH_CHECK();
   {
     WArgs a = {};
-    a.nex = 1; a.N = pf; a.K = d; a.ks = 1; a.gelu_r16 = 1;
+    a.nex = 1; a.N = pf; a.K = d; a.ks = 1;
     a.ex[0].w = (const h16x8*)ph[2 * order + 2]; a.ex[0].a = A; a.ex[0].lda = d;
     a.ex[0].bias = (const h16*)ph[2 * order + 3]; a.ex[0].out = G; a.ex[0].S = M;
-    if ((rc = launch_wide<E_GELU16>(a, pw.up, st))) return rc;
+    if ((rc = launch_wide<E_GELUF16>(a, pw.up, st))) return rc;
   }
   {
     WArgs a = {};
     a.nex = 1; a.N = d; a.K = pf; a.ks = pw.dn_ks;
     a.ex[0].w = (const h16x8*)ph[2 * order + 4]; a.ex[0].a = G; a.ex[0].lda = pf; a.ex[0].out = Pdn; a.ex[0].S = M;
-    if ((rc = launch_wide<E_PART>(a, PATH_SPLIT, st))) return rc;
+    if ((rc = launch_wide<E_PART>(a, path_split(M, d, 1, pw.dn_ks), st))) return rc;
   }
   PathOutArgs po = {};
   po.P = Pdn; po.bias = (const h16*)ph[2 * order + 5]; po.pred = (const h16*)pred; po.hsum = (h16*)hsum;

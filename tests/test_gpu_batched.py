@@ -20,7 +20,7 @@ import torch
 from conftest import rel_err, to64
 from chain_flow_amd.config import flownet
 from chain_flow_amd.drafter import Drafter
-from chain_flow_amd.head import ShortlistHead
+from chain_flow_amd.head import PathHead, ShortlistHead
 from chain_flow_amd.weights import make_weights, synthetic_context
 from oracle import beam as obeam
 from oracle import head as ohead
@@ -147,6 +147,57 @@ def test_grouped_head_and_batched_path_match_per_request_calls(cuda):
         e_req, e_or = rel_err(got, to64(hr)), rel_err(got, ref)
         print(f"  request {b}: batched path vs per-request {e_req:.2e}, vs oracle {e_or:.2e}", flush=True)
         assert e_req < 2e-3 and e_or < 2e-3, b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,M,nlive", [(2560, 17, 1), (2560, 128, 3), (5120, 64, 2), (5120, 97, 4)])
+def test_wide_path_residual_and_head_match_oracle(cuda, d, M, nlive):
+    """The path residual of 17-128 rows at the served widths, one to four live offsets, absent ancestors
+    mixed in, within fp16 rounding of the oracle; then the head with the markov bias over the rows it
+    returned: ids equal wherever the oracle's margin exceeds twice the logits' error bound (two ulps
+    and the fp32 dot product of each term, one ulp of their sum)."""
+    V, n, k = 2048, 1000, 4
+    cfg = flownet(d, layers=1, flow_steps=1)
+    g = torch.Generator().manual_seed(d + M)
+    mat = lambda r, c, s: (torch.randn(r, c, generator=g) * s).half()  # noqa: E731
+    W = {f"path_head.{p}": v for p, v in [
+        ("norm.weight", 1 + mat(1, d, 0.1)[0]), ("norm.bias", mat(1, d, 0.1)[0]),
+        ("mlp.0.weight", mat(2 * d, d, d ** -0.5)), ("mlp.0.bias", mat(1, 2 * d, 0.05)[0]),
+        ("mlp.3.weight", mat(d, 2 * d, (2 * d) ** -0.5)), ("mlp.3.bias", mat(1, d, 0.05)[0])]}
+    for j in range(cfg.path_order):
+        W[f"path_head.offset_proj.{j}.weight"] = mat(d, d, d ** -0.5)
+        W[f"path_head.offset_proj.{j}.bias"] = mat(1, d, 0.05)[0]
+    emb, lm, w1, w2 = mat(V, d, 0.5), mat(V, d, 3 * d ** -0.5), mat(V, 256, 1.0), mat(V, 256, 1 / 16)
+    sl = torch.randperm(V, generator=g)[:n].sort().values.to(torch.int32)
+    lastp = torch.randint(0, V, (M, cfg.path_order), generator=g, dtype=torch.int32)
+    lastp[1, 1:] = -1
+    lastp[M - 1, 2:] = -1
+    pred = torch.randn(d, generator=g).half()
+    print(f"[wide path] d={d} M={M} nlive={nlive}", flush=True)
+    ph = PathHead({n_: v.to(cuda) for n_, v in W.items()}, emb.to(cuda), cfg.path_order, cfg.path_ffn_multiplier, cuda)
+    head = ShortlistHead(lm.to(cuda), sl.to(cuda), w1.to(cuda), w2.to(cuda))
+    lastp_d = lastp.to(cuda)
+    rows = ph.hidden(lastp_d, nlive, pred.to(cuda))
+    vals, ids, _ = head.topk(rows, k, prev=lastp_d.view(-1), prev_stride=cfg.path_order)
+    torch.cuda.synchronize()
+    res = ohead.path_residual({n_: to64(v) for n_, v in W.items()}, to64(emb), lastp.long().numpy(), nlive,
+                              cfg.path_order)
+    got = to64(rows)
+    e = rel_err(got, ohead.r16(to64(pred)[None] + res, "fp16"))
+    print(f"  hidden {e:.2e}", flush=True)
+    assert e < 2e-3
+    s64 = sl.long().numpy()
+    lm64 = to64(lm)[s64]
+    prev = lastp[:, 0].long().numpy()
+    hw, mb = ohead.head_logits(got, lm64), ohead.markov_bias(to64(w1), to64(w2)[s64], prev)
+    ref = ohead.r16(hw + mb, "fp16")
+    bound = _bound(got, lm64, hw) + _bound(to64(w1)[prev], to64(w2)[s64], mb) + \
+        np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
+    order = np.argsort(-ref, axis=-1, kind="stable")[:, :k + 1]
+    near = np.take_along_axis(bound, order, -1).max(-1, keepdims=True)
+    ok = ohead.margins(ref, k) > 2 * near
+    print(f"  ids compared {ok.mean():.2f}", flush=True)
+    assert ok.any() and (ids.cpu().numpy()[ok] == order[:, :k][ok]).all()
 
 
 def _oracle(W, sl, cfg):

@@ -127,6 +127,38 @@ def test_path_residual_matches_oracle(cuda, nlive, M):
     assert rel_err(got, ref) < 2e-3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [4, 16, 17, 128])
+def test_path_gelu_is_torchs_erf_form(cuda, M):
+    """The path head's GELU bit for bit 0.5 x (1 + erf(x / sqrt 2)), its factors in float32 and their
+    product rounded once, for every finite fp16 x: a zero LayerNorm gain and a zero mlp.0 leave its bias
+    as the GELU's input, a unit mlp.3 passes the GELU on.  M: the narrow launches (up to 16 rows) and
+    the wide ones."""
+    d, pf, V = 512, 1024, 16
+    f16 = dict(dtype=torch.float16, device=cuda)
+    W = {"path_head.norm.weight": torch.zeros(d, **f16), "path_head.norm.bias": torch.zeros(d, **f16),
+         "path_head.mlp.0.weight": torch.zeros(pf, d, **f16), "path_head.mlp.0.bias": torch.zeros(pf, **f16),
+         "path_head.mlp.3.weight": torch.eye(d, pf, **f16), "path_head.mlp.3.bias": torch.zeros(d, **f16)}
+    for j in range(4):
+        W[f"path_head.offset_proj.{j}.weight"] = torch.zeros(d, d, **f16)
+        W[f"path_head.offset_proj.{j}.bias"] = torch.zeros(d, **f16)
+    ph = PathHead(W, torch.zeros(V, d, **f16), 4, 2, cuda)
+    x = torch.arange(-2 ** 15, 2 ** 15, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    x = x[torch.isfinite(x)].to(cuda)
+    lastp = torch.full((M, 4), -1, dtype=torch.int32, device=cuda)
+    pred = torch.zeros(d, **f16)
+    print(f"[path gelu] M={M} {len(x)} values", flush=True)
+    got = []
+    for part in x.split(d):
+        ph.b0[:len(part)] = part
+        got.append(ph.hidden(lastp, 1, pred)[:, :len(part)])
+    got = torch.cat(got, 1)
+    u = x.float()
+    # (the float64 product of two float32 factors is exact; numpy rounds it to fp16 in one step)
+    ref = (to64(0.5 * u) * to64(1.0 + torch.erf(u * 0.70710678118654752440))).astype(np.float16)
+    assert np.array_equal(got.cpu().numpy(), np.broadcast_to(ref, got.shape))
+
+
 def _np_chain_step(vals, ids, cum, lastp, sl, W):
     B = cum.shape[0]
     cand = (cum.reshape(B * W, 1) + vals).reshape(B, W * W)

@@ -4,6 +4,8 @@ from __future__ import annotations
 import re
 from pathlib import Path
 
+import pytest
+
 from chain_flow_amd import _lib
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "cfhip.h"
@@ -185,3 +187,22 @@ def test_flow_plan_flags_without_a_device():
     # 16 draft rows exceed the one-launch form's 8 rows a workgroup
     assert not plan_flags(flownet(640, layers=1, flow_steps=2, draft_length=16, chunk_size=8)) & X
 
+
+
+@pytest.mark.parametrize("d,M,order", [(512, 17, 4), (1024, 128, 4), (2560, 128, 4), (2560, 40, 3), (4096, 128, 3),
+                                       (4096, 200, 4), (5120, 17, 4), (5120, 128, 3), (5120, 97, 2)])
+def test_path_residual_splits_without_a_device(d, M, order):
+    """The k-splits of the path residual above 16 rows, read from its workspace: the first split of whole
+    128-column chunks that gives 256 workgroups of eight 16-column tiles.  They fix the order in which
+    the fp32 partials are added, and with it which of two nearly tied tokens a search depth returns."""
+    align = lambda n: (n + 255) // 256 * 256  # noqa: E731
+
+    def split(units, n, k):
+        legal = [s for s in range(1, k // 128 + 1) if k % s == 0 and k // s % 128 == 0]
+        return next((s for s in legal if units * (n // 128) * s >= 256), legal[-1])
+
+    rows, pf = min(M, 128), 2 * d
+    wide = (align(order * split(order, d, d) * rows * d * 4) + align(rows * d * 2) + align(rows * pf * 2)
+            + align(split(1, d, pf) * rows * d * 4))
+    L = _lib.lib()
+    assert L.cfh_path_ws_bytes(M, d, 2, order) == max(wide, L.cfh_path_ws_bytes(16, d, 2, order))
