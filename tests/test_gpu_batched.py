@@ -74,6 +74,29 @@ def test_gemm16_markov_equals_two_calls(cuda, M, n, d, stride):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [8, 128, 129, 256])
+def test_out_of_range_markov_parents_read_the_nearest_row(cuda, M):
+    """A parent of -1 (a beam row without one), and above 8 rows one past the table, at the row counts
+    where the head's launches change (GEMV, the bias in the GEMM, the bias before it): the same
+    result as the nearest row of w1, bit for bit."""
+    g = torch.Generator().manual_seed(M)
+    V, r, n, d = 600, 256, 500, 256
+    lm, w1, w2 = (torch.randn(V, x, generator=g).mul(0.1).half().to(cuda) for x in (d, r, r))
+    sl = torch.randperm(V, generator=g)[:n].sort().values.to(torch.int32).to(cuda)
+    head = ShortlistHead(lm, sl, w1, w2)
+    h = torch.randn(M, d, generator=g).half().to(cuda)
+    prev = torch.randint(0, V, (M,), generator=g, dtype=torch.int32)
+    prev[0], prev[M - 1] = -1, -1
+    if M > 8:
+        prev[M // 2] = V
+    print(f"[markov parents] M={M}", flush=True)
+    got = head.topk(h, 4, prev=prev.to(cuda))
+    ref = head.topk(h, 4, prev=prev.clamp(0, V - 1).to(cuda))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(got, ref))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,n,markov", [(9, 1024, True), (40, 1000, False), (160, 1024, True), (256, 777, True)])
 def test_gemm16_head_matches_oracle(cuda, M, n, markov):
     cfg, W, _ = _setup(n=n)
