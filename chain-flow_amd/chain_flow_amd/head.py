@@ -16,11 +16,14 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
     return t.to(torch.int32).contiguous()
 
 
-def _parents(prev: torch.Tensor, V: int) -> torch.Tensor:
-    """Markov parents as rows of a [V, r] table: an absent one (-1) reads row 0 and any other id out of
-    range the nearest row, as in the GEMM head's launch that gathers the rows itself."""
+def _parents(prev: torch.Tensor, w1: torch.Tensor) -> torch.Tensor:
+    """Markov parents as rows of the table w1 [V, r], on its device: an absent one (-1) reads row 0 and
+    any other id out of range the nearest row, as in the GEMM head's launch that gathers the rows
+    itself."""
+    if prev.device != w1.device:
+        raise RuntimeError(f"the markov parents are on {prev.device}, the table on {w1.device}")
     ids = prev if prev.dtype in (torch.int32, torch.int64) else prev.to(torch.long)
-    return ids.clamp(0, V - 1)
+    return ids.clamp(0, w1.shape[0] - 1)
 
 
 GEMV_ROWS = 8        # rows the GEMV head takes per launch; more go through the MFMA GEMM head
@@ -150,8 +153,9 @@ class ShortlistHead:
         h = h.contiguous()
         bias = None
         if prev is not None and self.w1 is not None and M <= GEMM_MARKOV_ROWS and self.r % 256 == 0:
-            ids32 = prev if prev.dtype == torch.int32 and prev.is_cuda and prev.stride(0) > 0 else \
-                _parents(prev, self.w1.shape[0]).to(h.device, torch.int32).contiguous()
+            # (int32 ids on the table's device go as they are: the launch clamps them)
+            ids32 = prev if prev.dtype == torch.int32 and prev.device == self.w1.device and prev.stride(0) > 0 else \
+                _parents(prev, self.w1).to(torch.int32).contiguous()
             vals, ids, lse = out
             ws = self.workspace(M, k, h.device)
             _lib.check(L.cfh_head_gemm16_markov_topk(
@@ -160,7 +164,7 @@ class ShortlistHead:
                 lse.data_ptr(), ws.data_ptr(), st), "cfh_head_gemm16_markov_topk")
             return vals, ids, lse
         if prev is not None and self.w1 is not None:
-            a = self.w1.index_select(0, _parents(prev, self.w1.shape[0])).contiguous()          # [M, r]
+            a = self.w1.index_select(0, _parents(prev, self.w1)).contiguous()          # [M, r]
             bias = torch.empty(M, self.n, dtype=torch.float16, device=h.device)
             w2img = self.image.data_ptr() + int(L.cfh_head_packed_bytes(self.n, self.d, 0))
             _lib.check(L.cfh_head_gemm16_topk(a.data_ptr(), M, self.r, w2img, self.n, None, 0, bias.data_ptr(),

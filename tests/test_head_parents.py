@@ -68,3 +68,14 @@ def test_absent_markov_parents_read_the_same_row_at_every_row_count(monkeypatch,
         assert np.array_equal(np.clip(got, 0, V - 1), last)
         if M > 256:
             assert np.array_equal(stub.rows.view(np.float16)[:, 0], want[:256])
+
+
+@pytest.mark.parametrize("M", [9, 128, 129, 256])
+def test_markov_parents_on_another_device_are_refused(monkeypatch, M):
+    """Parents that are not on the markov table's device never reach a launch (their address would not be
+    one of the launch's device)."""
+    head, stub = _head(monkeypatch)
+    prev = torch.zeros(M, dtype=torch.int32, device="meta")
+    with pytest.raises(RuntimeError, match="markov parents are on meta"):
+        head.topk(torch.zeros(M, D, dtype=torch.float16), 4, prev=prev)
+    assert stub.fused is None and stub.rows is None
