@@ -802,8 +802,9 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   // [2][MT*16][GKC], each row's 16-byte slots XOR-swizzled by the row's low 4 bits: the 16 rows
   // an MFMA operand read touches then fall on 16 different bank groups
   extern __shared__ __align__(16) uint16_t xs[];
-  // (the wave index read as a scalar keeps the image's pointers out of the vector registers)
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // MK: the wave index is read as a scalar and the lane's share added at each load, which keeps the two
+  // images' pointers out of the vector registers; with one image, lane pointers
+  const int wave = MK ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int ROWS = MT * 16, NG = GW / MS, MTW = MT / MS;
   static_assert(NG * MS == GW && MTW * MS == MT, "the row tiles and waves must split evenly");
   const int ng = wave % NG, mh = wave / NG;
@@ -815,7 +816,7 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   for (int t = 0; t < NT; ++t) {
     if constexpr (PK) {
       const int tile = min(tile0 + t, (a.n + 15) / 16 - 1);
-      wp[t] = (const bf16x8*)a.W + (size_t)tile * (a.d / 32) * 64;
+      wp[t] = (const bf16x8*)a.W + (size_t)tile * (a.d / 32) * 64 + (MK ? 0 : lane);
     } else {
       const int j = (tile0 + t) * 16 + (lane & 15);
       const int jc = j < a.n ? j : a.n - 1;
@@ -830,11 +831,12 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     wm[t] = MK ? (const bf16x8*)a.mw + (size_t)min(tile0 + t, (a.n + 15) / 16 - 1) * (a.r / 32) * 64 : nullptr;
-  // the fragment pointers of chunk c, the markov chunks counted before the head's
+  // k-step p's fragment of tile t in chunk c, the markov chunks counted before the head's (MK: wchunk is
+  // the chunk's scalar pointer)
   auto wchunk = [&](int c, int t) {
     return MK && c < nm ? wm[t] + c * GPF * KS : wp[t] + min(c - nm, nchunks - 1) * GPF * KS;
   };
-  const unsigned loff = PK ? lane * 16 : 0;           // the lane's share of an image fragment
+  const unsigned loff = MK ? lane * 16 : 0;
   auto frag = [&](const bf16x8* w, int p) __attribute__((always_inline)) {
     return wload<PK>((const bf16x8*)((const char*)(w + p * KS) + loff));
   };
@@ -847,8 +849,13 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
   for (int p = 0; p < GPF; ++p)
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      bqa[p][t] = frag(wchunk(0, t), p);
-      bqb[p][t] = frag(wchunk(1, t), p);
+      if constexpr (MK) {
+        bqa[p][t] = frag(wchunk(0, t), p);
+        bqb[p][t] = frag(wchunk(1, t), p);
+      } else {
+        bqa[p][t] = wload<PK>(wp[t] + p * KS);
+        bqb[p][t] = wload<PK>(wp[t] + (min(1, nchunks - 1) * GPF + p) * KS);
+      }
     }
   // x chunk: ROWS x 16 vectors of 8, XV a thread (vector idx = row*16 + v); branch-free, rows past
   // M repeat row M-1 (their products are never read), so the wait counts before the multiplies
@@ -903,8 +910,9 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
     if (MK && c + 1 < nm) load_xm(c + 1, xr);
     else load_x(min(c + 1 - nm, nchunks - 1), xr);
     const bf16x8* wn[NT];                             // chunk c + 2's fragments
+    const int cw = min(c + 2, nchunks - 1);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wn[t] = wchunk(c + 2, t);
+    for (int t = 0; t < NT; ++t) wn[t] = MK ? wchunk(c + 2, t) : nullptr;
     const uint16_t* xb = xs + (size_t)(c & 1) * ROWS * GKC + (size_t)(mh * MTW * 16 + (lane & 15)) * GKC;
 #pragma unroll
     for (int p = 0; p < GPF; ++p) {
@@ -929,7 +937,10 @@ __global__ void __launch_bounds__(GW * 64) k_head_gemm(GemmArgs a) {
       // keep the reloads here: the scheduler would otherwise sink them to the end of the chunk
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) bq[p][t] = frag(wn[t], p);
+      for (int t = 0; t < NT; ++t) {
+        if constexpr (MK) bq[p][t] = frag(wn[t], p);
+        else bq[p][t] = wload<PK>(wp[t] + (cw * GPF + p) * KS);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     store_x((c + 1) & 1, xr);
