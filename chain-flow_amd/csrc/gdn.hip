@@ -247,13 +247,16 @@ __device__ __forceinline__ uint16_t to_bf16(float x) { return __builtin_bit_cast
 //           LDS); a dot product is 8 products and a 16-lane DPP sum (no exchange between waves).
 //   k, q    GDN_VB steps of the path staged in LDS in the lanes' element order, the waves taking steps
 //           in turn.
-//   chains  GDN_CHAINS workgroups a (head, rows) take the leaves in turn, last (deepest) first.  A
-//           workgroup a node, most of which then end, took 28.3 us where this takes 18.7 (with the
-//           paired bf16 rounding below).
+//   chains  GDN_GRID workgroups in all, at least GDN_CHAINS a (head, rows), take the leaves in turn, last
+//           (deepest) first.  A workgroup a node, most of which then end, took 28.3 us where this takes
+//           18.7 (with the paired bf16 rounding below).  GDN_CHAINS alone left a bushy tree's leaves in
+//           line where few heads fill a part of the chip: 4 value heads, 200 roots 34.2 us, so 14.8; a
+//           random tree of 200 nodes 53 and 21; at 32 heads the two are one.
 // 41 nodes of that tree, 32 value heads, K = V = 128, bf16 states (44 MB): 46.4 -> 18.7 us.
 constexpr int GDN_VB = 16;   // path steps staged at once
 constexpr int GDN_VW = 4;    // waves of 16 value rows
-constexpr int GDN_CHAINS = 16;   // workgroups a (value head, 64 rows) that share the leaves
+constexpr int GDN_CHAINS = 16;   // workgroups a (value head, 64 rows) that share the leaves, at least
+constexpr int GDN_GRID = 1024;   // workgroups to fill the chip with where the heads are fewer
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
@@ -517,7 +520,7 @@ int cfh_gdn_tree_vllm(const void* mixed_qkv, const void* a, const void* b, const
   g.A_log = A_log; g.dt_bias = dt_bias; g.state = ssm_state; g.slots = node_slots; g.parent = parent;
   g.out = (uint16_t*)out; g.N = N; g.H = H; g.HV = HV; g.V = V; g.ld = 2 * H * K + HV * V;
   g.prefix = prefix_slot; g.nslots = nslots; g.status = status; g.l2norm = use_l2norm ? 1 : 0; g.scale = scale;
-  g.chains = std::min(N, GDN_CHAINS);
+  g.chains = std::min(N, std::max(GDN_CHAINS, GDN_GRID / (HV * (V / 64))));
   const long long blocks = (long long)g.chains * HV * (V / 64);
   if (state_bf16)
     hipLaunchKernelGGL(k_gdn_tree_vllm<uint16_t>, dim3((unsigned)blocks), dim3(64 * GDN_VW), 0, (hipStream_t)stream, g);
