@@ -283,7 +283,6 @@ __global__ void __launch_bounds__(TA_WAVES * 64) k_tree_attn(AttnArgs a) {
 // (value, first index), reduced over the wave and the workgroup (the larger value, then the lower
 // index) into ws[r][split]; the descent kernel then reduces a request's rows' slices in slice order.
 constexpr int ACC_SPLIT = 16;
-constexpr int ACC_LB = 8;    // 16-byte loads in flight a thread
 
 struct ArgPart { float v; int i; };
 
@@ -304,14 +303,14 @@ __global__ void __launch_bounds__(256) k_argmax_part(const u16* logits, int V, l
     // 8-element vectors over the aligned middle of [c0, c1), scalars at both ends
     const int v0 = (c0 + 7) / 8, v1 = c1 / 8;
     for (int j = c0 + threadIdx.x; j < min(c1, v0 * 8); j += blockDim.x) better(best, bix, ld2<IS_BF16>(row, j), j);
-    // ACC_LB vectors a thread in flight (one at a time: 16.5, so: 15.6 us for 164 rows x 248,320); past
-    // the slice the last vector again, which changes nothing
-    for (int u0 = v0 + threadIdx.x; u0 < v1; u0 += ACC_LB * 256) {
-      uint4 raw[ACC_LB];
+    // NB vectors a thread in flight from u0; past the slice the last vector again, which changes nothing
+    auto scan = [&](int u0, auto nb_c) __attribute__((always_inline)) {
+      constexpr int NB = decltype(nb_c)::value;
+      uint4 raw[NB];
 #pragma unroll
-      for (int b = 0; b < ACC_LB; ++b) raw[b] = *(const uint4*)(row + (size_t)min(u0 + b * 256, v1 - 1) * 8);
+      for (int b = 0; b < NB; ++b) raw[b] = *(const uint4*)(row + (size_t)min(u0 + b * 256, v1 - 1) * 8);
 #pragma unroll
-      for (int b = 0; b < ACC_LB; ++b) {
+      for (int b = 0; b < NB; ++b) {
         const int u = min(u0 + b * 256, v1 - 1);
         const u16* t = (const u16*)&raw[b];
 #pragma unroll
@@ -320,6 +319,16 @@ __global__ void __launch_bounds__(256) k_argmax_part(const u16* logits, int V, l
           if (v > best) { best = v; bix = u * 8 + e; }   // increasing index within a thread: > keeps the first
         }
       }
+    };
+    // eight at a time (164 rows x 248,320, whose slices have 7.6 a thread: one at a time 16.5 us, so 15.6);
+    // the last ones of a slice, or a narrower slice, as the least of 1, 2, 4 and 8 that holds them (the
+    // accept of 48 x 41 rows x 32,000, 1 a thread: always eight 80 us, so 35)
+    for (int u = v0; u + (int)threadIdx.x < v1; u += 8 * 256) {
+      const int left = (v1 - u + 255) / 256, u0 = u + (int)threadIdx.x;   // left: the same in every thread
+      if (left > 4) scan(u0, std::integral_constant<int, 8>{});
+      else if (left > 2) scan(u0, std::integral_constant<int, 4>{});
+      else if (left > 1) scan(u0, std::integral_constant<int, 2>{});
+      else scan(u0, std::integral_constant<int, 1>{});
     }
     for (int j = max(v1 * 8, v0 * 8) + threadIdx.x; j < c1; j += blockDim.x) better(best, bix, ld2<IS_BF16>(row, j), j);
   } else {
