@@ -321,8 +321,7 @@ __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
   const int S = min(Ssg, St - r0), C = min(Csg, Ct - c0);
   if (S <= 0 || C <= 0) return;                      // (a subgroup past the group's requests)
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  // this thread's first column of B_h (every context row of the subgroup), in flight before the
-  // scores; a block of more than XT columns gives the thread further columns XT apart
+  // this thread's CV columns of B_h (every context row of the subgroup), in flight before the scores
   typedef h16 hv __attribute__((ext_vector_type(CV)));
   const int cpb = d / a.nb, n = cb * cpb + min(t * CV, cpb - CV);
   const h16* Bbase = a.Bf[e] + ((size_t)h * Ct + c0) * d;
@@ -377,9 +376,9 @@ __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
   }
   __syncthreads();
   // this thread's columns of P_h B_h
+  if (t * CV >= cpb) return;
+  float* oh = a.out[e] + ((size_t)h * St + r0) * d + n;
   if constexpr (CV == 4) {
-    if (t * CV >= cpb) return;
-    float* oh = a.out[e] + ((size_t)h * St + r0) * d + n;
     // rows [ra, rb) over context rows [LO, LO + NC)
     auto rows = [&](int ra, int rb, auto lo, auto nc) __attribute__((always_inline)) {
       constexpr int LO = decltype(lo)::value, NC = decltype(nc)::value;
@@ -400,25 +399,15 @@ __global__ void __launch_bounds__(XT) k_xattn(XattArgs a) {
     } else {
       rows(0, S, std::integral_constant<int, 0>{}, std::integral_constant<int, CM>{});
     }
-    return;
   } else {
-    for (int cc = t; cc < cpb; cc += XT) {
-      const int nn = cb * cpb + cc;
-      float* oh = a.out[e] + ((size_t)h * St + r0) * d + nn;
-      float bf[CM];
-      if (cc == t) {
+    float bf[CM];
 #pragma unroll
-        for (int c = 0; c < CM; ++c) bf[c] = (float)bv[c][0];
-      } else {
+    for (int c = 0; c < CM; ++c) bf[c] = (float)bv[c][0];
+    for (int r = 0; r < S; ++r) {
+      float o = 0.f;
 #pragma unroll
-        for (int c = 0; c < CM; ++c) bf[c] = (float)Bbase[(size_t)min(c, C - 1) * d + nn];
-      }
-      for (int r = 0; r < S; ++r) {
-        float o = 0.f;
-#pragma unroll
-        for (int c = 0; c < CM; ++c) o += P[r][c] * bf[c];
-        oh[(size_t)r * d] = o;
-      }
+      for (int c = 0; c < CM; ++c) o += P[r][c] * bf[c];
+      oh[(size_t)r * d] = o;
     }
   }
 }
@@ -486,11 +475,10 @@ __global__ void __launch_bounds__(1024) k_xbias(XbiasArgs a) {
   }
 }
 
-// Column blocks per (expert, head) of XATT: the fewest that give each thread at most one column
-// (each block recomputes the head's scores, so more blocks only repeat that work); 0 if d has no
-// such split.
-// cv: columns a thread takes (each block recomputes its head's scores: the wide groups' many
-// subgroups already fill the chip, so there a thread takes four adjacent columns).
+// Column blocks per (expert, head) of XATT: the fewest that give each thread at most one share of cv
+// columns (each block recomputes the head's scores, so more blocks only repeat that work); 0 if d has
+// no such split.  cv: 1, or 4 adjacent columns in the wide groups, whose many subgroups already fill
+// the chip.
 int xattn_blocks(int d, int cv = 1) {
   for (int nb = 1; nb <= d; ++nb)
     if (d % nb == 0 && d / nb % cv == 0 && d / nb <= XT * cv) return nb;
@@ -504,9 +492,9 @@ int launch_xattn(const XattArgs& a, hipStream_t st) {
     const int Ssg = a.Ssg[e] > 0 ? a.Ssg[e] : a.S[e];
     if (Ssg > MAXR || (long long)a.nsg * Ssg < a.S[e]) return CFH_E_UNSUPPORTED;
   }
+  if ((a.cv != 1 && a.cv != 4) || a.d % a.nb || a.d / a.nb % a.cv || a.d / a.nb > XT * a.cv) return CFH_E_UNSUPPORTED;
   const dim3 grid((unsigned)(a.nex * a.H * a.nsg * a.nb));
   if (a.cv == 4) {
-    if (a.d / a.nb % 4 || a.d / a.nb > 4 * XT) return CFH_E_UNSUPPORTED;
     if (Csg <= 8) hipLaunchKernelGGL((k_xattn<8, 4>), grid, dim3(XT), 0, st, a);
     else hipLaunchKernelGGL((k_xattn<16, 4>), grid, dim3(XT), 0, st, a);
   } else {
@@ -1173,7 +1161,7 @@ int block_pass(const Plan& p, const cfh::ExpertLayout& L, const WS& w_all, const
   if (p.fold && !p.xblk) {
     XattArgs x = {};
     x.nex = nch; x.d = d; x.H = p.H; x.C = Cg; x.Cq = p.C; x.nb = p.xnb; x.scale = 1.0f / sqrtf((float)p.hd);
-    x.nsg = 1;
+    x.nsg = 1; x.cv = 1;
     const size_t per_l = (size_t)p.H * Cg * d;
     for (int c = 0; c < nch; ++c) {
       x.xn[c] = w.abuf[c]; x.A[c] = w.fa[c] + (size_t)l * per_l; x.Bf[c] = w.fb[c] + (size_t)l * per_l;
