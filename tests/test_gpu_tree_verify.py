@@ -158,3 +158,27 @@ def test_tree_greedy_accept_matches_oracle(cuda):
     assert np.array_equal(ln.cpu().numpy(), l_ref)
     assert np.array_equal(path.cpu().numpy(), p_ref) and np.array_equal(out.cpu().numpy(), o_ref)
     assert l_ref.max() >= 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [8, 1000, 32768, 32776, 65536, 65544, 131072, 131088, 262144, 262160, 300008, 1003])
+def test_greedy_accept_argmax_at_slice_widths(cuda, V):
+    """The row arg-max over vocabularies whose 16 slices hold up to 1, 2, 4, 8 or more 16-byte vectors a
+    thread, at those edges (1003: rows no vector load can read): the first of a row's largest values,
+    wherever it lies, and with the value repeated after it."""
+    B = 48
+    g = torch.Generator().manual_seed(V)
+    logits = torch.randn(B * 2, V, generator=g).clamp(-4, 4).bfloat16()
+    at = torch.randint(0, V, (B * 2,), generator=g)
+    at[:4] = torch.tensor([0, V - 1, V // 2, V // 16])
+    rows = torch.arange(B * 2)
+    logits[rows, at] = 5.0
+    logits[rows[::3], at[::3] + ((V - 1 - at[::3]) // 2)] = 5.0        # again, later in the row
+    print(f"[accept argmax] V={V}", flush=True)
+    cu_draft, cu_rows = np.arange(1, B + 1), np.arange(2, 2 * B + 1, 2)
+    draft = at[0::2].numpy().copy()                                      # every draft is its root's token
+    out, path, ln = tree_greedy_accept(logits.to(cuda), cu_draft, cu_rows, draft, np.full(B, -1), 1)
+    torch.cuda.synchronize()
+    ref = otv.greedy_descent(otv.first_argmax(logits.float().numpy()), cu_draft, cu_rows, draft, np.full(B, -1), 1)
+    assert np.array_equal(otv.first_argmax(logits.float().numpy()), at.numpy())
+    assert all(np.array_equal(x.cpu().numpy(), y) for x, y in zip((out, path, ln), ref))
