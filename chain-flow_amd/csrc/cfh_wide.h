@@ -344,7 +344,9 @@ int wide_check(const WArgs& a, WShape s, int S_max, int ch = WCH) {
 
 // Shape of a full-K launch of `units` units of `tiles` column tiles: the one with the least rounds of
 // 256 workgroups x (tiles a workgroup + 4), the 4 for what a workgroup costs whatever its tiles (its
-// start, the staging of the rows); the last listed on ties.
+// start, the staging of the rows); the last listed on ties.  Without the 4, flow passes (4 layers, 2
+// steps) take 2.89 ms where this takes 2.67 (16 requests, d = 4096), 3.33 where 3.25 (8, d = 5120), 1.32
+// where 1.23 (16, d = 2048); at d = 1024 up to 16 requests and in the latent drafter the two agree.
 WShape wide_shape_for(int tiles, int units) {
   constexpr int CUS = 256;
   WShape best = {};
@@ -361,7 +363,11 @@ WShape wide_shape_for(int tiles, int units) {
   return best;
 }
 
-// k-splits of a split-K launch: the most workgroups up to one a CU.
+// k-splits of a split-K launch: the most workgroups up to one a CU (the operand buffers of more than 64
+// rows leave room for one).  The first split to give 256, whose last round is then nearly empty, takes
+// 4.35 ms where this takes 3.97 (flow pass of 4 layers and 2 steps, 16 requests, d = 5120: 160 workgroups
+// for 320), 1.27 where 1.17 (8 requests, d = 2560) and 1.76 where 1.66 (16 requests of the latent
+// drafter); at d = 1024, 2048 and 4096 the two agree.
 int wide_ks(int N, int K, int units, WShape s) {
   constexpr int CUS = 256;
   int best = 0;
